@@ -11,6 +11,22 @@ constexpr int NY = 16;
 constexpr int NP = 20;      // padded tile extent (nghost = 2)
 constexpr int NC = NP * NP; // cells per padded tile
 
+// Order of a tile's 400 cells in device memory, per variable: the interior,
+// row by row (cells 0..255: whole 128-byte lines, which the padded rows are
+// not), then ghost layer 1 and ghost layer 2 as 4 sides x 16 positions each
+// (left, right, bottom, top; 256..319 and 320..383), then the 16 corner cells.
+// What the stages read and write is then contiguous: interior, interior plus
+// layer 1, or the ring.  (i, j) = -1..18; host buffers keep the padded rows
+// (launch_transpose converts).
+constexpr int tile_cell(int i, int j) {
+  if (i >= 1 && i <= NX && j >= 1 && j <= NY) return (j - 1) * NX + (i - 1);
+  const bool xout = i < 1 || i > NX, yout = j < 1 || j > NY;
+  if (xout && yout) return 384 + 4 * (j < 1 ? j + 1 : j - NY + 1) + (i < 1 ? i + 1 : i - NX + 1);
+  const int layer = xout ? (i < 1 ? 1 - i : i - NX) : (j < 1 ? 1 - j : j - NY);
+  const int side = xout ? (i < 1 ? 0 : 1) : (j < 1 ? 2 : 3);
+  return 256 + (layer - 1) * 64 + side * 16 + (xout ? j : i) - 1;
+}
+
 // Ghost-segment op kinds.  A destination block's non-corner ghost ring is 4
 // sides x 2 halves ("segments", seg = side*2 + half; side 0 left, 1 right,
 // 2 bottom, 3 top; half 0 covers positions 1..8, half 1 positions 9..16).
@@ -188,7 +204,10 @@ int launch_meshops(const wx_params *P, int neq, const MeshOp *ops, int nops, dou
 // Performs the n copies described in d (itself in mapped host memory), one
 // launch for all: a kernel reads the pinned staging directly.
 int launch_h2d(const CopyDesc *d, int n, hipStream_t stream);
-int launch_transpose(int neq, int cap, const double *src, double *dst, int to_fortran, int ld,
+// mode 0: Fortran layout (src) to cap device tiles (dst, from block 1 on); 1:
+// back; in place (src == dst), cap tiles from the given one on: 2: padded host
+// rows to the device's cell order, 3: back.
+int launch_transpose(int neq, int cap, const double *src, double *dst, int mode, int ld,
                      hipStream_t stream);
 
 // The OUTFYB compat mode of src/boundaryI.f90:87 is in effect: a bottom box

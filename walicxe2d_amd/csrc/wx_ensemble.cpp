@@ -570,8 +570,10 @@ int grp_basegrid(EnsGroup *e, int32_t inst, const double *uroots, int32_t nroots
   e->binfo_dev[inst] = 0;
   e->shadow[inst].valid = false;
   const size_t bytes = (size_t)(nroots + 1) * e->tile() * sizeof(double);
-  HIPCHK(hipMemcpyAsync(e->cur_u() + (size_t)e->slotbase[inst] * e->tile(), uroots, bytes, hipMemcpyHostToDevice,
-                        e->stream));
+  double *u = e->cur_u() + (size_t)e->slotbase[inst] * e->tile();
+  HIPCHK(hipMemcpyAsync(u, uroots, bytes, hipMemcpyHostToDevice, e->stream));
+  rc = launch_transpose(e->neq, nroots + 1, u, u, 2, 0, e->stream);
+  if (rc) return fail(rc, "reorder launch failed");
   HIPCHK(hipStreamSynchronize(e->stream));
   return WX_OK;
 }
@@ -634,11 +636,7 @@ int grp_download(EnsGroup *e, int32_t inst, double *u) {
   int rc = check_inst(e, inst);
   if (rc) return rc;
   if (!u) return fail(WX_EARG, "null buffer");
-  const size_t bytes = (size_t)(e->m[inst].nbmax + 1) * e->tile() * sizeof(double);
-  HIPCHK(hipMemcpyAsync(u, e->cur_u() + (size_t)e->slotbase[inst] * e->tile(), bytes, hipMemcpyDeviceToHost,
-                        e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));
-  return WX_OK;
+  return tiles_to_host(e, e->cur_u() + (size_t)e->slotbase[inst] * e->tile(), (size_t)e->m[inst].nbmax + 1, e->neq, u);
 }
 
 int grp_get_tree(EnsGroup *e, int32_t inst, int32_t *lp, int32_t *leaf, int32_t *icoord, int32_t ld,

@@ -570,6 +570,8 @@ int wx_upload(wx_ctx *c, const double *u, int32_t layout, const int32_t *lp, con
   if (layout == WX_LAYOUT_BLOCK) {
     const size_t n = (size_t)(nbmax + 1) * c->neq * NC;
     HIPCHK(hipMemcpyAsync(c->cur_u(), u, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    rc = launch_transpose(c->neq, nbmax + 1, c->cur_u(), c->cur_u(), 2, 0, c->stream);
+    if (rc) return fail(rc, "reorder launch failed");
   } else if (layout == WX_LAYOUT_FORTRAN) {
     if (ld > c->cap) return fail(WX_EARG, "ld %d exceeds capacity %d", ld, c->cap);
     const size_t n = (size_t)ld * c->neq * NC;
@@ -604,7 +606,7 @@ int wx_download(wx_ctx *c, double *u, double *prim, int32_t layout, int32_t ld_i
   for (int pass = 0; pass < 2; ++pass) {
     double *dst = pass == 0 ? u : prim;
     if (!dst) continue;
-    const double *src = c->cur_u();
+    double *src = c->cur_u();
     if (pass == 1) {
       if ((rc = c->dScratch.ensure((size_t)(c->cap + 1) * c->neq * NC))) return rc;
       rc = launch_calcprim(c->dP.ptr, c->neq, c->nbmax, c->cur_u(), c->dScratch.ptr, c->stream);
@@ -612,8 +614,7 @@ int wx_download(wx_ctx *c, double *u, double *prim, int32_t layout, int32_t ld_i
       src = c->dScratch.ptr;
     }
     if (layout == WX_LAYOUT_BLOCK) {
-      HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-      HIPCHK(hipStreamSynchronize(c->stream));
+      if ((rc = tiles_to_host(c, src, (size_t)c->nbmax + 1, c->neq, dst))) return rc;
     } else if (layout == WX_LAYOUT_FORTRAN) {
       const int ld = ld_in > 0 ? ld_in : c->nbmax;
       if (ld < c->nbmax || ld > c->cap) return fail(WX_EARG, "download: ld %d outside [nbmax %d, capacity %d]", ld, c->nbmax, c->cap);
@@ -765,6 +766,8 @@ int wx_basegrid(wx_ctx *c, const double *uroots, int32_t nroots) {
   c->pc_stale = true;
   const size_t n = (size_t)(nroots + 1) * c->neq * NC;
   HIPCHK(hipMemcpyAsync(c->cur_u(), uroots, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  rc = launch_transpose(c->neq, nroots + 1, c->cur_u(), c->cur_u(), 2, 0, c->stream);
+  if (rc) return fail(rc, "reorder launch failed");
   HIPCHK(hipStreamSynchronize(c->stream));
   return WX_OK;
 }

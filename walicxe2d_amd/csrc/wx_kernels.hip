@@ -1,9 +1,10 @@
 // wx_kernels.hip -- gfx950 kernels of the Walicxe-2D hot path.
 //
 // Data layout in HBM: one padded 20x20 tile per variable per block,
-// [id][var][j][i] with i fastest, id = the reference's block ID.  Every
-// kernel below assigns one 256-thread workgroup (4 wave64) to one leaf
-// block and stages the tile in LDS.
+// [id][var][cell], id = the reference's block ID, the cells in the order of
+// tile_cell (interior, ghost layer 1, ghost layer 2, corners).  Every kernel
+// below assigns one workgroup to one leaf block and stages the tile in LDS,
+// there as padded rows (IDX).
 //
 // One step (src/tstep.f90:4-126) is three launches over the leaf list:
 //   k_stageA      Uⁿ -> U^{n+1/2} interior (first-order fluxes, dt/2)
@@ -23,6 +24,7 @@
 namespace wx {
 
 __device__ __forceinline__ int IDX(int i, int j) { return (j + 1) * NP + (i + 1); }
+__device__ __forceinline__ int INT(int i, int j) { return (j - 1) * NX + (i - 1); }   // tile_cell of an interior cell
 
 // Queue entry of workgroup b in a one-entry-per-workgroup launch of G
 // workgroups.  The hardware deals workgroups to the 8 XCDs round robin
@@ -46,7 +48,7 @@ template <int NEQ>
 __device__ __forceinline__ void src_cell(const wx_params *__restrict__ p, const double *__restrict__ A,
                                          const BlockRec *__restrict__ binfo, int b, int i, int j,
                                          bool imposed, double vjet, double *v) {
-  const double *t = A + (size_t)b * NEQ * NC + IDX(i, j);
+  const double *t = A + (size_t)b * NEQ * NC + INT(i, j);   // gathers read interiors
 #pragma unroll
   for (int k = 0; k < NEQ; ++k) v[k] = t[k * NC];
   if (imposed) {
@@ -131,6 +133,18 @@ __device__ __forceinline__ void ghost_coords(int side, int layer, int pos, int &
   const bool xside = side < 2;
   i = xside ? edge : pos;
   j = xside ? pos : edge;
+}
+
+// (i, j) of cell c < 320 of a tile's device order: the interior, then ghost
+// layer 1.
+__device__ __forceinline__ void tile_ij(int c, int &i, int &j) {
+  if (c < 256) {
+    i = c % 16 + 1;
+    j = c / 16 + 1;
+  } else {
+    const int g = c - 256;
+    ghost_coords(g >> 4, 1, (g & 15) + 1, i, j);
+  }
 }
 
 // Flux sweep shared by both stages.  prim: LDS tile [NEQ][NC].  F: x-faces
@@ -243,23 +257,22 @@ __global__ __launch_bounds__(BS, PERSIST ? 1 : 8) void k_stageA(const wx_params 
   const wx_params *__restrict__ p = P + L.inst;
   DevScalars *__restrict__ S = Sa + L.inst;
   const double *ub = U + (size_t)L.id * NEQ * NC;
-  // rows j = 0..17 are one contiguous range [NP, 19*NP) of every variable.
-  // Under DMC the pressure of cells 0..17 is the one the last cooling left
-  // (the reference's primit, src/coolingdmc.f90:27-38 and
+  // the interior and ghost layer 1 are one contiguous range of every
+  // variable.  Under DMC the pressure of cells 0..17 is the one the last
+  // cooling left (the reference's primit, src/coolingdmc.f90:27-38 and
   // src/tstep.f90:27-36), not the one u gives back.
   const bool carried = Pc && p->cooling == 2;
   const double *pcb = carried ? Pc + (size_t)L.id * NC : nullptr;
-  for (int c = threadIdx.x; c < 18 * NP; c += blockDim.x) {
+  for (int c = threadIdx.x; c < 320; c += blockDim.x) {
     double uu[NEQ], q[NEQ], T;
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) uu[k] = ub[k * NC + NP + c];
+    for (int k = 0; k < NEQ; ++k) uu[k] = ub[k * NC + c];
     uprim<NEQ>(p, q, uu, T);
-    if (carried) {
-      const int col = c % NP;
-      if (col >= 1 && col <= 18) q[3] = pcb[NP + c];
-    }
+    if (carried) q[3] = pcb[c];
+    int i, j;
+    tile_ij(c, i, j);
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) prim[k * NC + NP + c] = q[k];
+    for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(i, j)] = q[k];
   }
   __syncthreads();
   int err = flux_sweep<NEQ, 1>(p, prim, F, G);
@@ -274,10 +287,10 @@ __global__ __launch_bounds__(BS, PERSIST ? 1 : 8) void k_stageA(const wx_params 
     double *qb = Q + (size_t)L.id * NEQ * NC;
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) {
-      double v = ub[k * NC + IDX(i, j)] - dtdx * (F[k * 272 + (j - 1) * 17 + i] - F[k * 272 + (j - 1) * 17 + i - 1])
+      double v = ub[k * NC + threadIdx.x] - dtdx * (F[k * 272 + (j - 1) * 17 + i] - F[k * 272 + (j - 1) * 17 + i - 1])
                  - dtdy * (G[k * 272 + j * 16 + (i - 1)] - G[k * 272 + (j - 1) * 16 + (i - 1)]);
       if (p->cylindrical) v = v + dtm * Sc[k];
-      qb[k * NC + IDX(i, j)] = v;
+      qb[k * NC + threadIdx.x] = v;
     }
   }
   if (err) atomicOr(&S->err, WX_EHLLC);
@@ -321,20 +334,20 @@ __global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, 
   const int gt = BS >= 384 ? tid - 256 : tid;
   const bool ghost = gt >= 0 && gt < 128;
   const int side = gt >> 5, layer = ((gt >> 4) & 1) + 1, pos = (gt & 15) + 1;
+  const bool keep1 = (p->compat & 2) && p->bc[2] == 0;   // lb_outfyb
   int2 op = make_int2(0, 0);
   if (ghost) op = ops[r * 8 + side * 2 + ((pos - 1) >> 3)];
   double u0[NEQ];
   if (tid < 256) {
-    const int i = tid % 16 + 1, j = tid / 16 + 1;
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) u0[k] = ub[k * NC + IDX(i, j)];
+    for (int k = 0; k < NEQ; ++k) u0[k] = ub[k * NC + tid];
   }
   // interior of U^{n+1/2} (imposed when the block is in the source list)
   if (tid < 256) {
     const int i = tid % 16 + 1, j = tid / 16 + 1;
     double uu[NEQ], q[NEQ], T;
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) uu[k] = qb[k * NC + IDX(i, j)];
+    for (int k = 0; k < NEQ; ++k) uu[k] = qb[k * NC + tid];
     if (imp && in_jet(p, L.level, L.icx, L.icy, i, j)) jet_state<NEQ>(p, vjet, uu);
     uprim<NEQ>(p, q, uu, T);
 #pragma unroll
@@ -369,7 +382,7 @@ __global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, 
       int ri, rj;
       ghost_coords(g >> 4, 1, (g & 15) + 1, ri, rj);
 #pragma unroll
-      for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(ri, rj)] = ub[k * NC + IDX(ri, rj)];
+      for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(ri, rj)] = ub[k * NC + 256 + g];
     }
     __syncthreads();
   }
@@ -394,15 +407,16 @@ __global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, 
   // reads of other cells were from the tile in LDS)
   if (tid < 256)
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) ub[k * NC + IDX(i, j)] = un[k];
+    for (int k = 0; k < NEQ; ++k) ub[k * NC + tid] = un[k];
   // the ring of U^{n+1/2} goes to its own tile's ring in the U^{n+1/2}
   // buffer (Qring is Q: this launch reads only interiors of Q), where the
   // fill leaves layer 2 as the step's final value (src/tstep.f90:85 copies
-  // up's ring into u; boundaryI rewrites layer 1 only)
-  if (ghost) {
-    double *rb = Qring + (size_t)b * NEQ * NC;
+  // up's ring into u; boundaryI rewrites layer 1, except the segments that
+  // the OUTFYB mode's list leaves to the carried values)
+  if (ghost && (layer == 2 || keep1)) {
+    double *rb = Qring + (size_t)b * NEQ * NC + 256 + (layer - 1) * 64 + side * 16 + pos - 1;
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) rb[k * NC + IDX(gi, gj)] = gh[k];
+    for (int k = 0; k < NEQ; ++k) rb[k * NC] = gh[k];
   }
   if (err) atomicOr(&S->err, WX_EHLLC);
   __syncthreads();   // the next queue entry reuses the LDS tiles
@@ -594,19 +608,6 @@ __device__ void cool_surrogate(const wx_params *__restrict__ p, SurDev *__restri
   }
 }
 
-// Cell c of the fill's per-cell passes: c < 256 the interior cell
-// (c % 16 + 1, c / 16 + 1); 256 <= c < 320 the layer-1 ghost that thread
-// c - 256 gathers (side (c - 256) / 16, position (c - 256) % 16 + 1).
-__device__ __forceinline__ void cool_cell(int c, int &i, int &j) {
-  if (c < 256) {
-    i = c % 16 + 1;
-    j = c / 16 + 1;
-  } else {
-    const int g = c - 256;
-    ghost_coords(g >> 4, 1, (g & 15) + 1, i, j);
-  }
-}
-
 // Waves per SIMD the plain one-entry-per-workgroup fill is compiled for: 5
 // caps it at 96 VGPRs (nothing spilled on its hot path), which measured
 // faster than 4 waves at 109 VGPRs (16.8 vs 17.8 ns per block on the
@@ -660,7 +661,7 @@ __global__ __launch_bounds__(BS, (SUR ? 2 : (PERSIST ? 1024 / BS : kFillWaves)))
     const int i = c % 16 + 1, j = c / 16 + 1;
     double uu[NEQ];
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) uu[k] = ib[k * NC + IDX(i, j)];
+    for (int k = 0; k < NEQ; ++k) uu[k] = ib[k * NC + c];
     if (imp && in_jet(p, L.level, L.icx, L.icy, i, j)) jet_state<NEQ>(p, vjet, uu);
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(i, j)] = uu[k];
@@ -680,7 +681,7 @@ __global__ __launch_bounds__(BS, (SUR ? 2 : (PERSIST ? 1024 / BS : kFillWaves)))
       ghost_gather<NEQ>(p, Uin, binfo, op, b, L.level, L.icx, L.icy, side, 1, pos, vjet, g);
     } else {
 #pragma unroll
-      for (int k = 0; k < NEQ; ++k) g[k] = ob[k * NC + IDX(gi, gj)];
+      for (int k = 0; k < NEQ; ++k) g[k] = ob[k * NC + 256 + gt];
       if (imp && in_jet(p, L.level, L.icx, L.icy, gi, gj)) jet_state<NEQ>(p, vjet, g);
     }
 #pragma unroll
@@ -697,7 +698,7 @@ __global__ __launch_bounds__(BS, (SUR ? 2 : (PERSIST ? 1024 / BS : kFillWaves)))
         double v[NEQ];
         jet_state<NEQ>(p, vjet, v);
 #pragma unroll
-        for (int k = 0; k < NEQ; ++k) ob[k * NC + IDX(gi, gj)] = v[k];
+        for (int k = 0; k < NEQ; ++k) ob[k * NC + 320 + g] = v[k];
       }
     }
   // cooling over cells 0..n+1 (src/coolingh.f90:19-20, src/coolingdmc.f90:23-24)
@@ -724,18 +725,18 @@ __global__ __launch_bounds__(BS, (SUR ? 2 : (PERSIST ? 1024 / BS : kFillWaves)))
   auto cool_pass = [&](auto cool) {
     for (int c = tid; c < 320; c += blockDim.x) {
       int i, j;
-      cool_cell(c, i, j);
+      tile_ij(c, i, j);
       double uu[NEQ];
 #pragma unroll
       for (int k = 0; k < NEQ; ++k) uu[k] = tile[k * NC + IDX(i, j)];
       const double pcool = cool(uu);
 #pragma unroll
-      for (int k = 0; k < NEQ; ++k) ob[k * NC + IDX(i, j)] = uu[k];
+      for (int k = 0; k < NEQ; ++k) ob[k * NC + c] = uu[k];
       double q[NEQ], T;
       uprim<NEQ>(p, q, uu, T);
       if (mode == 2) {
         q[3] = pcool;
-        if (Pc) Pc[(size_t)L.id * NC + IDX(i, j)] = pcool;
+        if (Pc) Pc[(size_t)L.id * NC + c] = pcool;
       }
 #pragma unroll
       for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(i, j)] = q[k];
@@ -789,11 +790,11 @@ __global__ __launch_bounds__(256) void k_blockstat(const wx_params *__restrict__
     const int i = c % 18, j = c / 18;
     double uu[NEQ], q[NEQ], T;
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) uu[k] = ub[k * NC + IDX(i, j)];
+    for (int k = 0; k < NEQ; ++k) uu[k] = ub[k * NC + tile_cell(i, j)];
     uprim<NEQ>(p, q, uu, T);
     if (carried) {
-      if (init) pcb[IDX(i, j)] = q[3];
-      else q[3] = pcb[IDX(i, j)];
+      if (init) pcb[tile_cell(i, j)] = q[3];
+      else q[3] = pcb[tile_cell(i, j)];
     }
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(i, j)] = q[k];
@@ -909,119 +910,76 @@ __global__ __launch_bounds__(256) void k_gather_flags(QueueRef q, const int32_t 
 // ---------------------------------------------------------------------
 // admesh data ops: src/refine.f90:30-42 (injection over the padded block)
 // and src/coarse.f90:182-366 (MPIP branch: 2x2 means incl. ghosts, then
-// outer ghost copies).  One workgroup per op.
+// outer ghost copies), and the statistics of the new leaf.  One workgroup per
+// new leaf, one thread per cell of its padded tile: a mesh change has a few
+// ops, so the launch is a chain of latencies (the op from host memory, the
+// source cells, the tile) and takes each once; with 256 threads, the copies
+// and the statistics reading the source separately and the outer ghosts
+// copied by one thread per variable it took 10.6 us against 7.5 for the few
+// ops of a step of the 64x16-root jet.
 template <int NEQ>
-__global__ __launch_bounds__(256) void k_meshops(const wx_params *__restrict__ P, const MeshOp *__restrict__ ops,
+__global__ __launch_bounds__(512) void k_meshops(const wx_params *__restrict__ P, const MeshOp *__restrict__ ops,
                                                  double *__restrict__ U, double *__restrict__ stat,
                                                  int8_t *__restrict__ flag, double *__restrict__ Pc) {
   // workgroup 4 * o + s: son s of a refine op o; a coarse op's dad is done
   // by its first workgroup
   const MeshOp op = ops[blockIdx.x >> 2];
-  const int part = blockIdx.x & 3;
+  const int s = blockIdx.x & 3;
+  const bool refine = op.kind == 0;
+  if (!refine && s != 0) return;
+  const int son = s == 0 ? op.s1 : s == 1 ? op.s2 : s == 2 ? op.s3 : op.s4;
+  const int dst = refine ? son : op.a;
+  const wx_params *__restrict__ p = P + op.inst;
+  double *pcb = (Pc && p->cooling == 2) ? Pc + (size_t)dst * NC : nullptr;
+  __shared__ double d[NEQ * NC];   // the new leaf's primitives, for its statistics
   const int tid = threadIdx.x;
-  __shared__ double d[NEQ * NC];   // coarse: the dad tile; then a tile of primitives for the statistics
-  if (op.kind == 0) {
-    const double *pb = U + (size_t)op.a * NEQ * NC;
-    const int s = part;
-    const int son = s == 0 ? op.s1 : s == 1 ? op.s2 : s == 2 ? op.s3 : op.s4;
-    double *sb = U + (size_t)son * NEQ * NC;
-    for (int cc = tid; cc < NC; cc += blockDim.x) {
-      const int i = cc % NP - 1, j = cc / NP - 1;
-      const int si = (i + 1) / 2 + ((s & 1) ? NX / 2 : 0);
-      const int sj = (j + 1) / 2 + ((s & 2) ? NY / 2 : 0);
+  if (tid < NC) {
+    const int i = tid % NP - 1, j = tid / NP - 1;
+    double uu[NEQ];
+    if (refine) {
+      const double *pb = U + (size_t)op.a * NEQ * NC +
+                         tile_cell((i + 1) / 2 + ((s & 1) ? NX / 2 : 0), (j + 1) / 2 + ((s & 2) ? NY / 2 : 0));
 #pragma unroll
-      for (int k = 0; k < NEQ; ++k) sb[k * NC + cc] = pb[k * NC + IDX(si, sj)];
-    }
-    // statistics of the son from its cells 0..17, which are the parent's
-    // cells it was injected from (read back from the parent, not the son);
-    // under DMC its carried pressure starts from them (src/refine.f90:231-258
-    // recomputes the sons' primit)
-    const wx_params *__restrict__ p = P + op.inst;
-    double *pcb = (Pc && p->cooling == 2) ? Pc + (size_t)son * NC : nullptr;
-    if (!stat && !pcb) return;
-    for (int c = tid; c < 18 * 18; c += blockDim.x) {
-      const int i = c % 18, j = c / 18;
-      const int si = (i + 1) / 2 + ((s & 1) ? NX / 2 : 0);
-      const int sj = (j + 1) / 2 + ((s & 2) ? NY / 2 : 0);
-      double uu[NEQ], q[NEQ], T;
-#pragma unroll
-      for (int k = 0; k < NEQ; ++k) uu[k] = pb[k * NC + IDX(si, sj)];
-      uprim<NEQ>(p, q, uu, T);
-      if (pcb) pcb[IDX(i, j)] = q[3];
-#pragma unroll
-      for (int k = 0; k < NEQ; ++k) d[k * NC + IDX(i, j)] = q[k];
-    }
-    if (!stat) return;
-    __syncthreads();
-    LeafRec L{};
-    L.id = son;
-    L.level = op.level;
-    L.inst = op.inst;
-    block_stats<NEQ>(p, d, L, stat, flag, FlagOut{nullptr, nullptr, nullptr, 0});
-  } else {
-    if (part != 0) return;
-    const int sons[4] = {op.s1, op.s2, op.s3, op.s4};
-    // start from the current dad tile (corners the rules below do not set)
-    const double *dbg = U + (size_t)op.a * NEQ * NC;
-    for (int c = tid; c < NEQ * NC; c += blockDim.x) d[c] = dbg[c];
-    __syncthreads();
-    // dad cells (0..17)^2 from the four sons: son s covers i in [is0, is1]
-    for (int c = tid; c < 18 * 18; c += blockDim.x) {
-      const int i = c % 18, j = c / 18;
-      const int sx = (i <= NX / 2) ? 0 : 1, sy = (j <= NY / 2) ? 0 : 1;
-      const int s = sx + 2 * sy;
-      const int li = i - sx * (NX / 2), lj = j - sy * (NY / 2);
-      const double *sb = U + (size_t)sons[s] * NEQ * NC;
-      const int i1 = 2 * li - 1, j1 = 2 * lj - 1;
+      for (int k = 0; k < NEQ; ++k) uu[k] = pb[k * NC];
+    } else {
+      // dad cells 0..17 from the four sons (son covers half of either
+      // direction); the outermost cells take their neighbour's value: the
+      // copies of src/coarse.f90:349-358, applied in order, leave every one
+      // of them with the nearest cell of 0..17
+      const int ci = min(max(i, 0), NX + 1), cj = min(max(j, 0), NY + 1);
+      const int sx = (ci <= NX / 2) ? 0 : 1, sy = (cj <= NY / 2) ? 0 : 1;
+      const int from = sy ? (sx ? op.s4 : op.s3) : (sx ? op.s2 : op.s1);
+      const int i1 = 2 * (ci - sx * (NX / 2)) - 1, j1 = 2 * (cj - sy * (NY / 2)) - 1;
+      const double *sb = U + (size_t)from * NEQ * NC;
+      const int c00 = tile_cell(i1, j1), c10 = tile_cell(i1 + 1, j1), c01 = tile_cell(i1, j1 + 1),
+                c11 = tile_cell(i1 + 1, j1 + 1);
 #pragma unroll
       for (int k = 0; k < NEQ; ++k)
-        d[k * NC + IDX(i, j)] = 0.25 * (((sb[k * NC + IDX(i1, j1)] + sb[k * NC + IDX(i1 + 1, j1)])
-                                        + sb[k * NC + IDX(i1, j1 + 1)]) + sb[k * NC + IDX(i1 + 1, j1 + 1)]);
+        uu[k] = 0.25 * (((sb[k * NC + c00] + sb[k * NC + c10]) + sb[k * NC + c01]) + sb[k * NC + c11]);
     }
-    __syncthreads();
-    // outer ghost copies (src/coarse.f90:349-358), same order
-    if (tid < NEQ) {
-      double *dk = d + tid * NC;
-      for (int j = -1; j <= NY + 2; ++j) dk[IDX(-1, j)] = dk[IDX(0, j)];
-      for (int j = -1; j <= NY + 2; ++j) dk[IDX(NX + 2, j)] = dk[IDX(NX + 1, j)];
-      for (int i = -1; i <= NX + 2; ++i) dk[IDX(i, -1)] = dk[IDX(i, 0)];
-      for (int i = -1; i <= NX + 2; ++i) dk[IDX(i, NY + 2)] = dk[IDX(i, NY + 1)];
-      dk[IDX(-1, -1)] = dk[IDX(0, -1)];
-      dk[IDX(NX + 2, -1)] = dk[IDX(NX + 2, 0)];
-      dk[IDX(-1, NY + 2)] = dk[IDX(-1, NY + 1)];
-      dk[IDX(NX + 2, NY + 2)] = dk[IDX(NX + 1, NY + 2)];
-    }
-    __syncthreads();
-    double *db = U + (size_t)op.a * NEQ * NC;
-    for (int c = tid; c < NEQ * NC; c += blockDim.x) db[c] = d[c];
-    // statistics of the dad: primitives of its cells 0..17 in place; under
-    // DMC its carried pressure starts from them (src/coarse.f90:178, 360
-    // recompute the dad's primit)
-    const wx_params *__restrict__ p = P + op.inst;
-    double *pcb = (Pc && p->cooling == 2) ? Pc + (size_t)op.a * NC : nullptr;
-    if (!stat && !pcb) return;
-    __syncthreads();
-    for (int c = tid; c < 18 * 18; c += blockDim.x) {
-      const int i = c % 18, j = c / 18;
-      double uu[NEQ], q[NEQ], T;
+    double *db = U + (size_t)dst * NEQ * NC + tile_cell(i, j);
 #pragma unroll
-      for (int k = 0; k < NEQ; ++k) uu[k] = d[k * NC + IDX(i, j)];
+    for (int k = 0; k < NEQ; ++k) db[k * NC] = uu[k];
+    // primitives of cells 0..17; under DMC the carried pressure starts from
+    // them (src/refine.f90:231-258, src/coarse.f90:178, 360 recompute primit)
+    if ((stat || pcb) && i >= 0 && i <= NX + 1 && j >= 0 && j <= NY + 1) {
+      double q[NEQ], T;
       uprim<NEQ>(p, q, uu, T);
-      if (pcb) pcb[IDX(i, j)] = q[3];
+      if (pcb) pcb[tile_cell(i, j)] = q[3];
 #pragma unroll
       for (int k = 0; k < NEQ; ++k) d[k * NC + IDX(i, j)] = q[k];
     }
-    if (!stat) return;
-    __syncthreads();
-    LeafRec L{};
-    L.id = op.a;
-    L.level = op.level;
-    L.inst = op.inst;
-    block_stats<NEQ>(p, d, L, stat, flag, FlagOut{nullptr, nullptr, nullptr, 0});
   }
+  if (!stat) return;
+  __syncthreads();
+  LeafRec L{};
+  L.id = dst;
+  L.level = op.level;
+  L.inst = op.inst;
+  block_stats<NEQ>(p, d, L, stat, flag, FlagOut{nullptr, nullptr, nullptr, 0});
 }
 
-// Layout transposes between [id][var][j][i] and the reference's
+// Layout transposes between the device's tiles and the reference's
 // u(nb, ieq, i, j) with nb fastest (ld = number of block rows).
 template <int NEQ>
 __global__ void k_transpose(int cap, const double *__restrict__ src, double *__restrict__ dst,
@@ -1032,13 +990,32 @@ __global__ void k_transpose(int cap, const double *__restrict__ src, double *__r
       // t enumerates the Fortran array: nb fastest
       const size_t nb = t % cap, r = t / cap;
       const size_t k = r % NEQ, cell = r / NEQ;     // cell = (i+1) + 20*(j+1)
-      dst[t] = src[((nb + 1) * NEQ + k) * NC + cell];
+      dst[t] = src[((nb + 1) * NEQ + k) * NC + tile_cell((int)(cell % NP) - 1, (int)(cell / NP) - 1)];
     } else {
       const size_t cell = t % NC, r = t / NC;
       const size_t k = r % NEQ, id = r / NEQ;       // id 0..cap-1 -> block id+1
-      dst[((id + 1) * NEQ + k) * NC + cell] = src[(cell * NEQ + k) * (size_t)ld + id];
+      dst[((id + 1) * NEQ + k) * NC + tile_cell((int)(cell % NP) - 1, (int)(cell / NP) - 1)] =
+          src[(cell * NEQ + k) * (size_t)ld + id];
     }
   }
+}
+
+// The cells of one tile variable per 128 threads reordered in place, between
+// padded host rows and the device's order.
+__global__ __launch_bounds__(256) void k_reorder(size_t ntile, double *__restrict__ u, int to_rows) {
+  __shared__ double t[2][NC];
+  const int h = threadIdx.x >> 7, l = threadIdx.x & 127;
+  const size_t v = (size_t)blockIdx.x * 2 + h;
+  double *b = u + v * NC;
+  if (v < ntile)
+    for (int c = l; c < NC; c += 128) t[h][c] = b[c];
+  __syncthreads();
+  if (v < ntile)
+    for (int c = l; c < NC; c += 128) {
+      const int d = tile_cell(c % NP - 1, c / NP - 1);
+      if (to_rows) b[c] = t[h][d];
+      else b[d] = t[h][c];
+    }
 }
 
 template <int NEQ>
@@ -1163,7 +1140,7 @@ int launch_gather_flags(QueueRef q, const int32_t *inst_off, int grid, const int
 int launch_meshops(const wx_params *P, int neq, const MeshOp *ops, int nops, double *U, double *stat, int8_t *flag,
                    double *Pc, hipStream_t stream) {
   if (nops <= 0) return WX_OK;
-  WX_DISPATCH(neq, hipLaunchKernelGGL(k_meshops<N>, dim3(4 * nops), dim3(256), 0, stream, P, ops, U, stat, flag, Pc));
+  WX_DISPATCH(neq, hipLaunchKernelGGL(k_meshops<N>, dim3(4 * nops), dim3(512), 0, stream, P, ops, U, stat, flag, Pc));
   return hip_status();
 }
 
@@ -1196,8 +1173,15 @@ int launch_h2d(const CopyDesc *d, int n, hipStream_t stream) {
   return hip_status();
 }
 
-int launch_transpose(int neq, int cap, const double *src, double *dst, int to_fortran, int ld, hipStream_t stream) {
-  WX_DISPATCH(neq, hipLaunchKernelGGL(k_transpose<N>, dim3(1024), dim3(256), 0, stream, cap, src, dst, to_fortran, ld));
+int launch_transpose(int neq, int cap, const double *src, double *dst, int mode, int ld, hipStream_t stream) {
+  if (mode >= 2) {   // in place, cap tiles
+    if (src != dst) return WX_EARG;
+    const size_t ntile = (size_t)cap * neq;
+    if (ntile == 0) return WX_OK;
+    hipLaunchKernelGGL(k_reorder, dim3((unsigned)((ntile + 1) / 2)), dim3(256), 0, stream, ntile, dst, mode == 3);
+    return hip_status();
+  }
+  WX_DISPATCH(neq, hipLaunchKernelGGL(k_transpose<N>, dim3(1024), dim3(256), 0, stream, cap, src, dst, mode, ld));
   return hip_status();
 }
 

@@ -257,4 +257,15 @@ void WorkerPool::run(int n, const std::function<void(int)> &fn) {
   n_ = 0;
 }
 
+int tiles_to_host(Runtime *r, double *tiles, size_t ntile, int neq, double *host) {
+  int rc = launch_transpose(neq, (int)ntile, tiles, tiles, 3, 0, r->stream);
+  if (rc) return fail(rc, "reorder launch failed");
+  const hipError_t e1 = hipMemcpyAsync(host, tiles, ntile * neq * NC * sizeof(double), hipMemcpyDeviceToHost, r->stream);
+  rc = launch_transpose(neq, (int)ntile, tiles, tiles, 2, 0, r->stream);   // back, whatever the copy did
+  const hipError_t e2 = hipStreamSynchronize(r->stream);
+  if (rc) return fail(rc, "reorder launch failed");
+  if (e1 != hipSuccess || e2 != hipSuccess) return fail(WX_EHIP, "download copy failed");
+  return WX_OK;
+}
+
 }  // namespace wx

@@ -188,6 +188,11 @@ const void *stage_inplace(Runtime *r, const void *src, size_t bytes);
 // Launches the round's copies and records the buffer's event.
 int stage_end(Runtime *r);
 void prof_collect(Runtime *r);
+// ntile device tiles from `tiles` on to host memory as padded rows: reordered
+// in place, copied and ordered back, so that no second buffer is needed.
+// Returns when the copy is done.
+int tiles_to_host(Runtime *r, double *tiles, size_t ntile, int neq, double *host);
+
 int prof_report(Runtime *r, int32_t enable, double *ms, int64_t *counts, int32_t n);
 
 // Events around the launches of its scope on stream s (the runtime's own
