@@ -65,6 +65,42 @@ def test_gradient_matches_reference():
             k += n
 
 
+
+@pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 16384, 16449])
+def test_gradient_batch_sizes(n):
+    """The gradient at the edges of a workgroup's 64 samples and of the
+    256 workgroups that share a batch (16 384 samples are one pass of them):
+    FP32 sums of bf16 products against the same in 64 bits."""
+    m = _random_model(30 + n)
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(n, 4)).astype(np.float32)
+    t = rng.normal(size=(n, 2)).astype(np.float32)
+    loss, g = S.grad(m, x, t, w=(1.0, 0.5))
+    lr, gr = M.loss_and_grad(m.theta.astype(np.float64), x.astype(np.float64), t.astype(np.float64),
+                             w=(1.0, 0.5), round_bf16=True)
+    assert abs(loss - lr) <= 1e-3 * lr
+    assert np.abs(g - gr).max() <= 2e-2 * np.abs(gr).max()
+
+
+def test_training_wraps_around_the_data():
+    """Steps whose batch runs over the end of the data: the loss of each step
+    is that of the rows it names, on parameters that follow the reference."""
+    m = _random_model(7)
+    rng = np.random.default_rng(8)
+    n, batch, steps = 100, 65, 4
+    x = rng.normal(size=(n, 4)).astype(np.float32)
+    t = rng.normal(size=(n, 2)).astype(np.float32)
+    th, mm, vv, want = m.theta.astype(np.float64), 0.0, 0.0, []
+    for k in range(steps):
+        idx = (k * batch + np.arange(batch)) % n
+        loss, g = M.loss_and_grad(th, x[idx].astype(np.float64), t[idx].astype(np.float64), w=(1.0, 1.0), round_bf16=True)
+        want.append(loss)
+        mm, vv = 0.9 * mm + 0.1 * g, 0.999 * vv + 0.001 * g * g
+        th = th - 1e-4 * (mm / (1 - 0.9 ** (k + 1))) / (np.sqrt(vv / (1 - 0.999 ** (k + 1))) + 1e-8)
+    hist = S.train_steps(m, x, t, batch, steps, 1e-4, 1e-4)
+    assert np.allclose(hist, want, rtol=2e-3)
+
+
 def test_adam_step_matches_reference():
     m = _random_model(5)
     rng = np.random.default_rng(6)

@@ -20,29 +20,22 @@ namespace wx {
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ uint16_t f2bf(float f) {   // round to nearest even
-  uint32_t u = __float_as_uint(f);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+// To bf16, round to nearest even (v_cvt_pk_bf16_f32: two values an instruction).
+typedef __bf16 bf16x2h __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t f2bf_pk(float a, float b) {
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2h));
 }
+__device__ __forceinline__ uint16_t f2bf(float f) { return (uint16_t)f2bf_pk(f, f); }
 
 __device__ __forceinline__ bf16x4 pack4(float a, float b, float c, float d) {
-  bf16x4 r;
-  r[0] = (short)f2bf(a);
-  r[1] = (short)f2bf(b);
-  r[2] = (short)f2bf(c);
-  r[3] = (short)f2bf(d);
-  return r;
+  const uint2 v = make_uint2(f2bf_pk(a, b), f2bf_pk(c, d));
+  return __builtin_bit_cast(bf16x4, v);
 }
 
 __device__ __forceinline__ bf16x4 ld4(const uint16_t *p) {   // 4 consecutive bf16 (8-byte aligned)
-  const uint2 v = *reinterpret_cast<const uint2 *>(p);
-  bf16x4 r;
-  r[0] = (short)(v.x & 0xFFFF);
-  r[1] = (short)(v.x >> 16);
-  r[2] = (short)(v.y & 0xFFFF);
-  r[3] = (short)(v.y >> 16);
-  return r;
+  return __builtin_bit_cast(bf16x4, *reinterpret_cast<const uint2 *>(p));
 }
 
 __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
@@ -50,26 +43,19 @@ __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
 }
 
 
-// SiLU and its derivative with the hardware exp2 and reciprocal (1 ulp each).
+// SiLU with the hardware exp2 and reciprocal (1 ulp each).
 __device__ __forceinline__ float sigm(float z) { return __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
 __device__ __forceinline__ float silu(float z) { return z * sigm(z); }
-__device__ __forceinline__ float dsilu(float z) {
-  const float s = sigm(z);
-  return s * (1.f + z * (1.f - s));
-}
 
 // Forward pass of 16 samples by one wave.  x: B operand of layer 1 (lanes
 // 0-15 carry their sample's 4 standardised features, lanes 16-63 zeros).
 // w*: bf16 weights as in SurDev; b1..b4: the FP32 biases (global memory or
 // LDS copies).  Returns the D tile of layer 4 (rows 0, 1 = standardised
-// outputs of sample l in lanes l < 16).  If zs / as are given, the
-// pre-activations (D layout) and bf16 activations are kept for the backward
-// pass.
+// outputs of sample l in lanes l < 16).
 __device__ __forceinline__ f32x4 mlp_fwd16(const uint16_t *__restrict__ w1, const uint16_t *__restrict__ w2,
                                            const uint16_t *__restrict__ w3, const uint16_t *__restrict__ w4,
                                            const float *__restrict__ b1, const float *__restrict__ b2,
-                                           const float *__restrict__ b3, const float *__restrict__ b4, bf16x4 x,
-                                           f32x4 (*zs)[4] = nullptr, bf16x4 (*as)[4] = nullptr) {
+                                           const float *__restrict__ b3, const float *__restrict__ b4, bf16x4 x) {
   const int l = threadIdx.x & 63;
   const int r = l & 15, q = l >> 4;
   bf16x4 a[4];
@@ -80,29 +66,27 @@ __device__ __forceinline__ f32x4 mlp_fwd16(const uint16_t *__restrict__ w1, cons
     acc = mfma16(ld4(w1 + (16 * mt + r) * 16 + 4 * q), x, acc);
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] += b1[16 * mt + 4 * q + e];
-    if (zs) zs[0][mt] = acc;
     a[mt] = pack4(silu(acc[0]), silu(acc[1]), silu(acc[2]), silu(acc[3]));
-    if (as) as[0][mt] = a[mt];
   }
   // layers 2 and 3: 64 -> 64
 #pragma unroll
   for (int layer = 0; layer < 2; ++layer) {
     const uint16_t *__restrict__ w = layer == 0 ? w2 : w3;
     const float *__restrict__ b = layer == 0 ? b2 : b3;
-    bf16x4 an[4];
+    // the four output tiles side by side: independent matrix instructions
+    f32x4 acc[4];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) acc[mt] = mfma16(ld4(w + (16 * mt + r) * 64 + 16 * kt + 4 * q), a[kt], acc[mt]);
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt) acc = mfma16(ld4(w + (16 * mt + r) * 64 + 16 * kt + 4 * q), a[kt], acc);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] += b[16 * mt + 4 * q + e];
-      if (zs) zs[layer + 1][mt] = acc;
-      an[mt] = pack4(silu(acc[0]), silu(acc[1]), silu(acc[2]), silu(acc[3]));
-      if (as) as[layer + 1][mt] = an[mt];
+      for (int e = 0; e < 4; ++e) acc[mt][e] += b[16 * mt + 4 * q + e];
+      a[mt] = pack4(silu(acc[mt][0]), silu(acc[mt][1]), silu(acc[mt][2]), silu(acc[mt][3]));
     }
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) a[mt] = an[mt];
   }
   // layer 4: 64 -> 2 (rows padded to 16)
   f32x4 y = {0.f, 0.f, 0.f, 0.f};
@@ -116,10 +100,9 @@ __device__ __forceinline__ f32x4 mlp_fwd16(const uint16_t *__restrict__ w1, cons
 }
 
 // The forward pass with the weights and biases of a model in global memory.
-__device__ __forceinline__ f32x4 mlp_fwd16(const SurDev *__restrict__ M, bf16x4 x, f32x4 (*zs)[4] = nullptr,
-                                           bf16x4 (*as)[4] = nullptr) {
+__device__ __forceinline__ f32x4 mlp_fwd16(const SurDev *__restrict__ M, bf16x4 x) {
   return mlp_fwd16(M->w1, M->w2, M->w3, M->w4, M->theta + SUR_B1, M->theta + SUR_B2, M->theta + SUR_B3,
-                   M->theta + SUR_B4, x, zs, as);
+                   M->theta + SUR_B4, x);
 }
 
 // al = ALOSS / n^2 at (T, x_HII) from the table (bilinear in log10 T and

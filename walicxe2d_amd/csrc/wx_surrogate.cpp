@@ -154,15 +154,18 @@ int wx_sur_grad(const wx_sur_model *m, const float *x, const float *t, int64_t n
   if (rc) return rc;
   SurDev *M;
   if ((rc = model_on_device(S, m, nullptr, &M))) return rc;
-  float *dx, *dt, *dg, *dl;
+  float *dx, *dt, *dg, *dl, *part, *lpart;
+  SurTrain *W;
+  const int rows = sur_rows(n);
   if ((rc = S.alloc(&dx, (size_t)n * 4)) || (rc = S.alloc(&dt, (size_t)n * 2)) || (rc = S.alloc(&dg, SUR_NPARAM)) ||
-      (rc = S.alloc(&dl, 1)))
+      (rc = S.alloc(&dl, 1)) || (rc = S.alloc(&W, 1)) || (rc = S.alloc(&part, (size_t)rows * SUR_ROW)) ||
+      (rc = S.alloc(&lpart, rows)))
     return rc;
   HIPCHK(hipMemcpyAsync(dx, x, (size_t)n * 4 * sizeof(float), hipMemcpyHostToDevice, S.s));
   HIPCHK(hipMemcpyAsync(dt, t, (size_t)n * 2 * sizeof(float), hipMemcpyHostToDevice, S.s));
-  HIPCHK(hipMemsetAsync(dg, 0, SUR_NPARAM * sizeof(float), S.s));
-  HIPCHK(hipMemsetAsync(dl, 0, sizeof(float), S.s));
-  if ((rc = launch_sur_grad(M, dx, dt, 0, n, n, w0, w1, dg, dl, S.s))) return fail(rc, "gradient kernel failed");
+  if ((rc = launch_sur_packt(M, W, S.s)) || (rc = launch_sur_grad(M, W, dx, dt, 0, n, n, w0, w1, part, lpart, S.s)) ||
+      (rc = launch_sur_sum(M, part, lpart, rows, dg, dl, S.s)))
+    return fail(rc, "gradient kernel failed");
   HIPCHK(hipMemcpyAsync(grad, dg, SUR_NPARAM * sizeof(float), hipMemcpyDeviceToHost, S.s));
   float l = 0.f;
   HIPCHK(hipMemcpyAsync(&l, dl, sizeof(float), hipMemcpyDeviceToHost, S.s));
@@ -180,24 +183,26 @@ int wx_sur_train(wx_sur_model *m, const float *x, const float *t, int64_t n, int
   if (rc) return rc;
   SurDev *M;
   if ((rc = model_on_device(S, m, nullptr, &M))) return rc;
-  float *dx, *dt, *dg, *dm, *dv, *dl;
-  if ((rc = S.alloc(&dx, (size_t)n * 4)) || (rc = S.alloc(&dt, (size_t)n * 2)) || (rc = S.alloc(&dg, SUR_NPARAM)) ||
-      (rc = S.alloc(&dm, SUR_NPARAM)) || (rc = S.alloc(&dv, SUR_NPARAM)) || (rc = S.alloc(&dl, (size_t)steps + 1)))
+  float *dx, *dt, *dm, *dv, *dl, *part, *lpart;
+  SurTrain *W;
+  const int64_t nb = batch < n ? batch : n;
+  const int rows = sur_rows(nb);
+  if ((rc = S.alloc(&dx, (size_t)n * 4)) || (rc = S.alloc(&dt, (size_t)n * 2)) || (rc = S.alloc(&dm, SUR_NPARAM)) ||
+      (rc = S.alloc(&dv, SUR_NPARAM)) || (rc = S.alloc(&dl, (size_t)steps + 1)) || (rc = S.alloc(&W, 1)) ||
+      (rc = S.alloc(&part, (size_t)rows * SUR_ROW)) || (rc = S.alloc(&lpart, rows)))
     return rc;
   HIPCHK(hipMemcpyAsync(dx, x, (size_t)n * 4 * sizeof(float), hipMemcpyHostToDevice, S.s));
   HIPCHK(hipMemcpyAsync(dt, t, (size_t)n * 2 * sizeof(float), hipMemcpyHostToDevice, S.s));
   HIPCHK(hipMemsetAsync(dm, 0, SUR_NPARAM * sizeof(float), S.s));
   HIPCHK(hipMemsetAsync(dv, 0, SUR_NPARAM * sizeof(float), S.s));
   HIPCHK(hipMemsetAsync(dl, 0, ((size_t)steps + 1) * sizeof(float), S.s));
-  const int64_t nb = batch < n ? batch : n;
+  if ((rc = launch_sur_packt(M, W, S.s))) return fail(rc, "pack kernel");
   for (int k = 0; k < steps; ++k) {
     const double frac = steps > 1 ? (double)k / (double)(steps - 1) : 0.0;
     const float lr = (float)((double)lr0 * std::pow((double)lr1 / (double)lr0, frac));
     const int64_t off = (int64_t)(((__int128)k * nb) % n);
-    HIPCHK(hipMemsetAsync(dg, 0, SUR_NPARAM * sizeof(float), S.s));
-    if ((rc = launch_sur_grad(M, dx, dt, off, nb, n, w0, w1, dg, dl + k, S.s))) return fail(rc, "gradient kernel");
-    if ((rc = launch_sur_adam(M, dg, dm, dv, k + 1, lr, S.s))) return fail(rc, "adam kernel");
-    if ((rc = launch_sur_pack(M, S.s))) return fail(rc, "pack kernel");
+    if ((rc = launch_sur_grad(M, W, dx, dt, off, nb, n, w0, w1, part, lpart, S.s))) return fail(rc, "gradient kernel");
+    if ((rc = launch_sur_adam(M, W, part, lpart, rows, dm, dv, k + 1, lr, dl + k, S.s))) return fail(rc, "adam kernel");
   }
   HIPCHK(hipMemcpyAsync(m->theta, M->theta, sizeof m->theta, hipMemcpyDeviceToHost, S.s));
   if (loss_hist && steps > 0)

@@ -54,9 +54,25 @@ int launch_sur_pack(SurDev *M, hipStream_t stream);
 int launch_sur_altab(const wx_params *P, SurDev *M, hipStream_t stream);
 int launch_sur_feat(const SurDev *M, const double *in, int64_t n, float *f, float *cedt, hipStream_t stream);
 int launch_sur_infer(const SurDev *M, const float *x, int64_t n, float *y, hipStream_t stream);
-int launch_sur_grad(const SurDev *M, const float *x, const float *t, int64_t off, int64_t nbatch, int64_t ndata,
-                    float w0, float w1, float *grad, float *loss, hipStream_t stream);
-int launch_sur_adam(SurDev *M, const float *grad, float *m, float *v, int step, float lr, hipStream_t stream);
+// Training: transposed bf16 weights ([in][out]) for the backward pass.
+struct SurTrain {
+  alignas(16) uint16_t w2t[64 * 64], w3t[64 * 64], w4t[64 * 16];   // w4t: [in][out padded to 16]
+};
+// Rows of the gradient's partial sums: one per workgroup of 64 samples, at
+// most one workgroup per CU of the card; SUR_ROW floats apart.
+constexpr int SUR_ROW = 8832;
+constexpr int SUR_MAXROWS = 256;
+inline int sur_rows(int64_t nb) { return (int)((nb + 63) / 64 < SUR_MAXROWS ? (nb + 63) / 64 : SUR_MAXROWS); }
+int launch_sur_packt(const SurDev *M, SurTrain *W, hipStream_t stream);
+// Forward and backward of a batch: part[sur_rows(nb)][SUR_ROW], lpart[rows].
+int launch_sur_grad(const SurDev *M, const SurTrain *W, const float *x, const float *t, int64_t off, int64_t nbatch,
+                    int64_t ndata, float w0, float w1, float *part, float *lpart, hipStream_t stream);
+// The rows' sum as the gradient and the loss ...
+int launch_sur_sum(SurDev *M, const float *part, const float *lpart, int nrow, float *grad, float *loss,
+                   hipStream_t stream);
+// ... or as one Adam step of M (and of W's and M's bf16 copies).
+int launch_sur_adam(SurDev *M, SurTrain *W, const float *part, const float *lpart, int nrow, float *m, float *v,
+                    int step, float lr, float *loss, hipStream_t stream);
 int launch_cool_pairs(const wx_params *P, const double *in, int64_t n, double *out, hipStream_t stream);
 // host side (wx_surrogate.cpp)
 int sur_upload(SurDev *M, const wx_sur_model *m, const wx_params *P, hipStream_t stream);
