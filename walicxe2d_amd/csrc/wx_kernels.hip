@@ -497,82 +497,82 @@ __device__ void block_stats(const wx_params *__restrict__ p, const double *prim,
 // (src/coolingh.f90:249-250) evaluated with the tabulated loss; the energy
 // residual is the change of thermal energy (2 - y1) T1 that correction
 // makes, relative to the old thermal energy (2 - y0) T.
-// The network's weights and biases staged in LDS once per workgroup.
-struct SurLds {
-  uint16_t w1[64 * 16], w2[64 * 64], w3[64 * 64], w4[16 * 64];
-  float b[64 * 3 + 2];
-};
-
-template <bool SUR>
-struct SurSlot {
-  using type = SurLds;
-};
-template <>
-struct SurSlot<false> {
-  using type = char;
-};
-
-__device__ void sur_stage(const SurDev *__restrict__ M, SurLds *L) {
-  for (int t = threadIdx.x; t < 64 * 64 / 4; t += blockDim.x) {   // 8-byte chunks
-    reinterpret_cast<uint2 *>(L->w2)[t] = reinterpret_cast<const uint2 *>(M->w2)[t];
-    reinterpret_cast<uint2 *>(L->w3)[t] = reinterpret_cast<const uint2 *>(M->w3)[t];
-    if (t < 64 * 16 / 4) {
-      reinterpret_cast<uint2 *>(L->w1)[t] = reinterpret_cast<const uint2 *>(M->w1)[t];
-      reinterpret_cast<uint2 *>(L->w4)[t] = reinterpret_cast<const uint2 *>(M->w4)[t];
-    }
-  }
-  for (int t = threadIdx.x; t < 64; t += blockDim.x) {
-    L->b[t] = M->theta[SUR_B1 + t];
-    L->b[64 + t] = M->theta[SUR_B2 + t];
-    L->b[128 + t] = M->theta[SUR_B3 + t];
-  }
-  if (threadIdx.x < 2) L->b[192 + threadIdx.x] = M->theta[SUR_B4 + threadIdx.x];
-}
-
-template <int NEQ>
-__device__ void cool_surrogate(const wx_params *__restrict__ p, SurDev *__restrict__ M, const SurLds *W, double dts,
-                               double *tile) {
-  __shared__ float sx[324 * 4];
-  __shared__ float sy[324 * 2];
-  __shared__ float scedt[324];
-  __shared__ uint8_t sinh[324];
-  __shared__ unsigned int nfb;
+// A cell outside takes the exact routine in a pass of its own, over a list
+// of such cells: a wave that held one of them used to run it for all its cells.
+// Each cell is worked on by the thread that loaded it into the tile (cell
+// tid, then tid + BS), which also writes its cooled state to ob and its
+// primitives to the tile.  The inference reads every cell's features.
+template <int NEQ, int BS>
+__device__ __forceinline__ void cool_surrogate(const wx_params *__restrict__ p, SurDev *__restrict__ M, double dts,
+                                               double *tile, double *__restrict__ ob) {
+  constexpr int NWAVE = BS / 64, G = (20 + NWAVE - 1) / NWAVE;   // 20 groups of 16 cells
+  __shared__ bf16x4 sx[320];
+  __shared__ float sy[320 * 2];
+  __shared__ float scedt[320];      // ce dt of the tabulated relaxation; negative outside the hull
+  __shared__ double sT[320], sK[320];   // temperature, kinetic energy
+  __shared__ uint16_t list[320];
+  __shared__ uint32_t nfb;
   const int tid = threadIdx.x;
   if (tid == 0) nfb = 0u;
-  for (int c = tid; c < 324; c += blockDim.x) {
-    const int i = c % 18, j = c / 18;
+#pragma unroll
+  for (int n = 0; n < (320 + BS - 1) / BS; ++n) {
+    const int c = tid + n * BS;
+    if (c >= 320) break;
+    int i, j;
+    tile_ij(c, i, j);
     double uu[NEQ], q[NEQ], T;
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) uu[k] = tile[k * NC + IDX(i, j)];
     uprim<NEQ>(p, q, uu, T);
     float f[4], cedt;
-    sinh[c] = sur_features(M, uu[0], T, uu[4] / uu[0], dts, f, cedt) ? 1 : 0;
-    scedt[c] = cedt;
+    const bool in = sur_features(M, uu[0], T, uu[4] / uu[0], dts, f, cedt);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) sx[4 * c + k] = (f[k] - M->in_mu[k]) / M->in_sig[k];
+    for (int k = 0; k < 4; ++k) f[k] = (f[k] - M->in_mu[k]) / M->in_sig[k];
+    sx[c] = pack4(f[0], f[1], f[2], f[3]);
+    scedt[c] = in ? cedt : -1.f;
+    sT[c] = T;
+    sK[c] = 0.5 * q[0] * (q[1] * q[1] + q[2] * q[2]);
   }
   __syncthreads();
   {
-    const int l = tid & 63, r = l & 15, qq = l >> 4;
-    for (int g = tid >> 6; g < 21; g += (int)(blockDim.x >> 6)) {   // 21 groups of 16 cover the 324 cells
-      const int c = 16 * g + r;
-      bf16x4 xb = {0, 0, 0, 0};
-      if (qq == 0 && c < 324) xb = pack4(sx[4 * c], sx[4 * c + 1], sx[4 * c + 2], sx[4 * c + 3]);
-      const f32x4 y = mlp_fwd16(W->w1, W->w2, W->w3, W->w4, W->b, W->b + 64, W->b + 128, W->b + 192, xb);
-      if (qq == 0 && c < 324) {
-        sy[2 * c] = y[0];
-        sy[2 * c + 1] = y[1];
+    const int l = tid & 63, r = l & 15, qq = l >> 4, w = tid >> 6;
+    bf16x4 xb[G];
+    f32x4 y[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int c = 16 * (w + NWAVE * g) + r;
+      xb[g] = bf16x4{0, 0, 0, 0};
+      if (qq == 0 && c < 320) xb[g] = sx[c];
+    }
+    mlp_fwd16<G>(M, xb, y);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int c = 16 * (w + NWAVE * g) + r;
+      if (qq == 0 && c < 320) {
+        sy[2 * c] = y[g][0];
+        sy[2 * c + 1] = y[g][1];
       }
     }
   }
   __syncthreads();
-  unsigned int mine = 0;
-  for (int c = tid; c < 324; c += blockDim.x) {
-    const int i = c % 18, j = c / 18;
-    double uu[NEQ], q[NEQ], T;
+  auto put = [&](int c, int i, int j, const double *uu) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < NEQ; ++k) ob[k * NC + c] = uu[k];
+    double q[NEQ], T;
+    uprim<NEQ>(p, q, uu, T);
+#pragma unroll
+    for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(i, j)] = q[k];
+  };
+#pragma unroll
+  for (int n = 0; n < (320 + BS - 1) / BS; ++n) {
+    const int c = tid + n * BS;
+    if (c >= 320) break;
+    int i, j;
+    tile_ij(c, i, j);
+    double uu[NEQ];
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) uu[k] = tile[k * NC + IDX(i, j)];
-    uprim<NEQ>(p, q, uu, T);
+    const double T = sT[c];
     const double y0 = uu[4] / uu[0];
     const float corr = sy[2 * c] * M->out_sig[0] + M->out_mu[0];
     const float dx = sy[2 * c + 1] * M->out_sig[1] + M->out_mu[1];
@@ -581,7 +581,8 @@ __device__ void cool_surrogate(const wx_params *__restrict__ p, SurDev *__restri
     y1 = dmax(y1, 0.0001);
     // the relaxation law with the tabulated loss, then the network's
     // correction log10(T1 / T1_table)
-    double tt = 10. + (T - 10.) * (double)__expf(-scedt[c]);
+    const float cedt = scedt[c];
+    double tt = 10. + (T - 10.) * (double)__expf(-cedt);
     tt = dmax(tt, 0.1 * T);
     tt = dmin(tt, 10. * T);
     tt = dmax(tt, 10.);
@@ -590,21 +591,29 @@ __device__ void cool_surrogate(const wx_params *__restrict__ p, SurDev *__restri
     t1 = dmin(t1, 10. * T);
     t1 = dmax(t1, 10.);
     const double resid = (2. - y1) * fabs(t1 - tt) / ((2. - y0) * T);
-    if (!sinh[c] || !(resid <= (double)M->tol)) {
-      atomic_h<NEQ>(p, dts, uu);
-      ++mine;
+    if (!(cedt >= 0.f) || !(resid <= (double)M->tol)) {
+      list[atomicAdd(&nfb, 1u)] = (uint16_t)c;
     } else {
       uu[4] = y1 * uu[0];
-      uu[3] = p->cv * (2. * uu[0] - uu[4]) * t1 / p->Tempsc + 0.5 * q[0] * (q[1] * q[1] + q[2] * q[2]);
+      uu[3] = p->cv * (2. * uu[0] - uu[4]) * t1 / p->Tempsc + sK[c];
+      put(c, i, j, uu);
     }
-#pragma unroll
-    for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(i, j)] = uu[k];
   }
-  if (mine) atomicAdd(&nfb, mine);
   __syncthreads();
+  const uint32_t n = nfb;
+  for (uint32_t k = tid; k < n; k += BS) {
+    const int c = list[k];
+    int i, j;
+    tile_ij(c, i, j);
+    double uu[NEQ];
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) uu[v] = tile[v * NC + IDX(i, j)];
+    atomic_h<NEQ>(p, dts, uu);
+    put(c, i, j, uu);
+  }
   if (tid == 0) {
-    atomicAdd(&M->fallbacks, (unsigned long long)nfb);
-    atomicAdd(&M->cells, 324ull);
+    if (n) atomicAdd(&M->fallbacks, (unsigned long long)n);
+    atomicAdd(&M->cells, 320ull);
   }
 }
 
@@ -616,7 +625,7 @@ __device__ void cool_surrogate(const wx_params *__restrict__ p, SurDev *__restri
 constexpr int kFillWaves = 5;
 
 template <int NEQ, bool SUR, int BS, bool PERSIST>
-__global__ __launch_bounds__(BS, (SUR ? 2 : (PERSIST ? 1024 / BS : kFillWaves))) void k_fillI_cool(const wx_params *__restrict__ P, QueueRef q,
+__global__ __launch_bounds__(BS, (SUR ? (PERSIST ? 2 : 1024 / BS) : (PERSIST ? 1024 / BS : kFillWaves))) void k_fillI_cool(const wx_params *__restrict__ P, QueueRef q,
                                                     const int2 *__restrict__ ops,
                                                     const BlockRec *__restrict__ binfo,
                                                     const double *__restrict__ Uin,
@@ -628,14 +637,6 @@ __global__ __launch_bounds__(BS, (SUR ? 2 : (PERSIST ? 1024 / BS : kFillWaves)))
                                                     SurDev *__restrict__ M,
                                                     double *__restrict__ Pc) {
   __shared__ double tile[NEQ * NC];
-  // the network in LDS, staged once per workgroup (no LDS without the surrogate)
-  __shared__ __align__(16) typename SurSlot<SUR>::type Wbuf;
-  SurLds *W = nullptr;
-  if constexpr (SUR) {
-    W = &Wbuf;
-    sur_stage(M, W);
-    __syncthreads();
-  }
   const int b0 = PERSIST ? (int)blockIdx.x : xcd_entry(blockIdx.x, gridDim.x);
   LeafRec Lnext = q.rec[min(b0, q.cap - 1)];
   const int nleaf = q.hdr->nleaf;
@@ -712,9 +713,7 @@ __global__ __launch_bounds__(BS, (SUR ? 2 : (PERSIST ? 1024 / BS : kFillWaves)))
   bool done = false;
   if constexpr (SUR && NEQ >= 5) {
     if (mode == 1) {
-      __syncthreads();   // the surrogate's cells are spread differently
-      cool_surrogate<NEQ>(p, M, W, S->dt * p->tsc, tile);
-      __syncthreads();
+      cool_surrogate<NEQ, BS>(p, M, S->dt * p->tsc, tile, ob);
       done = true;
     }
   }
@@ -756,7 +755,7 @@ __global__ __launch_bounds__(BS, (SUR ? 2 : (PERSIST ? 1024 / BS : kFillWaves)))
       cool_dmc<NEQ>(p, dts, uu, pcool);
       return pcool;
     });
-  } else {
+  } else if (!done) {
     cool_pass([](double *) { return 0.0; });
   }
   __syncthreads();

@@ -47,62 +47,74 @@ __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
 __device__ __forceinline__ float sigm(float z) { return __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
 __device__ __forceinline__ float silu(float z) { return z * sigm(z); }
 
-// Forward pass of 16 samples by one wave.  x: B operand of layer 1 (lanes
-// 0-15 carry their sample's 4 standardised features, lanes 16-63 zeros).
-// w*: bf16 weights as in SurDev; b1..b4: the FP32 biases (global memory or
-// LDS copies).  Returns the D tile of layer 4 (rows 0, 1 = standardised
-// outputs of sample l in lanes l < 16).
-__device__ __forceinline__ f32x4 mlp_fwd16(const uint16_t *__restrict__ w1, const uint16_t *__restrict__ w2,
-                                           const uint16_t *__restrict__ w3, const uint16_t *__restrict__ w4,
-                                           const float *__restrict__ b1, const float *__restrict__ b2,
-                                           const float *__restrict__ b3, const float *__restrict__ b4, bf16x4 x) {
+// Forward pass of G groups of 16 samples by one wave.  x[g]: B operand of
+// layer 1 (lanes 0-15 carry their sample's 4 standardised features, lanes
+// 16-63 zeros).  y[g]: the D tile of layer 4 (rows 0, 1 = standardised outputs
+// of sample l in lanes l < 16).  Each weight operand is loaded once, from
+// cache, and used by all groups.  With the weights staged in LDS by every
+// workgroup of the fill, read again for every group and kept at 47 KB of LDS
+// and two waves per SIMD, and with whole waves running the exact routine for
+// one cell outside, the fill took 139 us on 1 870 blocks; it takes 68.  A group
+// costs 48 exponentials and reciprocals per lane, about 2 300 SIMD cycles: 35
+// of the 68 us.
+template <int G>
+__device__ __forceinline__ void mlp_fwd16(const SurDev *__restrict__ M, const bf16x4 *x, f32x4 *y) {
   const int l = threadIdx.x & 63;
   const int r = l & 15, q = l >> 4;
-  bf16x4 a[4];
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  bf16x4 a[G][4], an[G][4];
+  auto activate = [&](const f32x4 &acc, const f32x4 &b) __attribute__((always_inline)) {
+    const f32x4 z = acc + b;
+    return pack4(silu(z[0]), silu(z[1]), silu(z[2]), silu(z[3]));
+  };
+  auto bias = [&](int off, int mt) __attribute__((always_inline)) {
+    return *reinterpret_cast<const f32x4 *>(M->theta + off + 16 * mt + 4 * q);
+  };
   // layer 1: K = 4 features padded to 16
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma16(ld4(w1 + (16 * mt + r) * 16 + 4 * q), x, acc);
+    const bf16x4 w = ld4(M->w1 + (16 * mt + r) * 16 + 4 * q);
+    const f32x4 b = bias(SUR_B1, mt);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] += b1[16 * mt + 4 * q + e];
-    a[mt] = pack4(silu(acc[0]), silu(acc[1]), silu(acc[2]), silu(acc[3]));
+    for (int g = 0; g < G; ++g) a[g][mt] = activate(mfma16(w, x[g], zero), b);
   }
   // layers 2 and 3: 64 -> 64
-#pragma unroll
-  for (int layer = 0; layer < 2; ++layer) {
-    const uint16_t *__restrict__ w = layer == 0 ? w2 : w3;
-    const float *__restrict__ b = layer == 0 ? b2 : b3;
-    // the four output tiles side by side: independent matrix instructions
-    f32x4 acc[4];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) acc[mt] = mfma16(ld4(w + (16 * mt + r) * 64 + 16 * kt + 4 * q), a[kt], acc[mt]);
+  auto hidden = [&](const uint16_t *__restrict__ w, int off, bf16x4(*in)[4], bf16x4(*out)[4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
+      const f32x4 b = bias(off, mt);
+      f32x4 acc[G];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[mt][e] += b[16 * mt + 4 * q + e];
-      a[mt] = pack4(silu(acc[mt][0]), silu(acc[mt][1]), silu(acc[mt][2]), silu(acc[mt][3]));
+      for (int g = 0; g < G; ++g) acc[g] = zero;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+        const bf16x4 wk = ld4(w + (16 * mt + r) * 64 + 16 * kt + 4 * q);
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g] = mfma16(wk, in[g][kt], acc[g]);
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) out[g][mt] = activate(acc[g], b);
+    }
+  };
+  hidden(M->w2, SUR_B2, a, an);
+  hidden(M->w3, SUR_B3, an, a);
+  // layer 4: 64 -> 2 (rows padded to 16)
+#pragma unroll
+  for (int g = 0; g < G; ++g) y[g] = zero;
+#pragma unroll
+  for (int kt = 0; kt < 4; ++kt) {
+    const bf16x4 wk = ld4(M->w4 + r * 64 + 16 * kt + 4 * q);
+#pragma unroll
+    for (int g = 0; g < G; ++g) y[g] = mfma16(wk, a[g][kt], y[g]);
+  }
+  if (q == 0) {
+    const float b0 = M->theta[SUR_B4], b1 = M->theta[SUR_B4 + 1];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      y[g][0] += b0;
+      y[g][1] += b1;
     }
   }
-  // layer 4: 64 -> 2 (rows padded to 16)
-  f32x4 y = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int kt = 0; kt < 4; ++kt) y = mfma16(ld4(w4 + r * 64 + 16 * kt + 4 * q), a[kt], y);
-  if (q == 0) {
-    y[0] += b4[0];
-    y[1] += b4[1];
-  }
-  return y;
-}
-
-// The forward pass with the weights and biases of a model in global memory.
-__device__ __forceinline__ f32x4 mlp_fwd16(const SurDev *__restrict__ M, bf16x4 x) {
-  return mlp_fwd16(M->w1, M->w2, M->w3, M->w4, M->theta + SUR_B1, M->theta + SUR_B2, M->theta + SUR_B3,
-                   M->theta + SUR_B4, x);
 }
 
 // al = ALOSS / n^2 at (T, x_HII) from the table (bilinear in log10 T and

@@ -59,19 +59,30 @@ __global__ __launch_bounds__(256) void k_sur_feat(const SurDev *__restrict__ M, 
   }
 }
 
-// Standardised inputs x[n][4] -> standardised outputs y[n][2].
+// Standardised inputs x[n][4] -> standardised outputs y[n][2]; a wave takes
+// 4 groups of 16 samples at a time.
 __global__ __launch_bounds__(256) void k_sur_infer(const SurDev *__restrict__ M, const float *__restrict__ x,
                                                    int64_t n, float *__restrict__ y) {
+  constexpr int G = 4;
   const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-  const int64_t ngroups = (n + 15) / 16;
-  for (int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); g < ngroups; g += (int64_t)gridDim.x * 4) {
-    const int64_t s = 16 * g + r;
-    bf16x4 xb = {0, 0, 0, 0};
-    if (q == 0 && s < n) xb = pack4(x[4 * s], x[4 * s + 1], x[4 * s + 2], x[4 * s + 3]);
-    const f32x4 yt = mlp_fwd16(M, xb);
-    if (q == 0 && s < n) {
-      y[2 * s] = yt[0];
-      y[2 * s + 1] = yt[1];
+  const int64_t nset = (n + 16 * G - 1) / (16 * G);
+  for (int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); b < nset; b += (int64_t)gridDim.x * 4) {
+    bf16x4 xb[G];
+    f32x4 yt[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int64_t s = 16 * (G * b + g) + r;
+      xb[g] = bf16x4{0, 0, 0, 0};
+      if (q == 0 && s < n) xb[g] = pack4(x[4 * s], x[4 * s + 1], x[4 * s + 2], x[4 * s + 3]);
+    }
+    mlp_fwd16<G>(M, xb, yt);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int64_t s = 16 * (G * b + g) + r;
+      if (q == 0 && s < n) {
+        y[2 * s] = yt[g][0];
+        y[2 * s + 1] = yt[g][1];
+      }
     }
   }
 }
@@ -403,7 +414,7 @@ int launch_sur_feat(const SurDev *M, const double *in, int64_t n, float *f, floa
 
 int launch_sur_infer(const SurDev *M, const float *x, int64_t n, float *y, hipStream_t stream) {
   if (n <= 0) return WX_OK;
-  hipLaunchKernelGGL(k_sur_infer, dim3(grid_for(n, 64)), dim3(256), 0, stream, M, x, n, y);
+  hipLaunchKernelGGL(k_sur_infer, dim3(grid_for(n, 256)), dim3(256), 0, stream, M, x, n, y);
   return hip_ok();
 }
 
