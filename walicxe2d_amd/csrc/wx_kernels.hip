@@ -17,6 +17,9 @@
 //                 buffer, and emits the next CFL partials and the refinement
 //                 flag of the block (fused timestep/criteria epilogue).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
+
 #include "wx_device.h"
 #include "wx_mlp.h"
 #include "wx_physics.h"
@@ -25,6 +28,16 @@ namespace wx {
 
 __device__ __forceinline__ int IDX(int i, int j) { return (j + 1) * NP + (i + 1); }
 __device__ __forceinline__ int INT(int i, int j) { return (j - 1) * NX + (i - 1); }   // tile_cell of an interior cell
+
+// threadIdx.x computed again from the wave's number (in a scalar register) and
+// the lane: two instructions each time instead of a vector register held, or
+// spilled, across a kernel whose budget is 64 of them.
+__device__ __forceinline__ int wave_of() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+__device__ __forceinline__ int tid_again(int wave) {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+  return wave * 64 + lane;
+}
 
 // Queue entry of workgroup b in a one-entry-per-workgroup launch of G
 // workgroups.  The hardware deals workgroups to the 8 XCDs round robin
@@ -58,7 +71,7 @@ __device__ __forceinline__ void src_cell(const wx_params *__restrict__ p, const 
 }
 
 template <int NEQ>
-__device__ void ghost_gather(const wx_params *__restrict__ p, const double *__restrict__ A,
+__device__ __forceinline__ void ghost_gather(const wx_params *__restrict__ p, const double *__restrict__ A,
                              const BlockRec *__restrict__ binfo, int2 op, int dst, int dlev,
                              int dicx, int dicy, int side, int layer, int pos, double vjet,
                              double *g) {
@@ -150,14 +163,14 @@ __device__ __forceinline__ void tile_ij(int c, int &i, int &j) {
 // Flux sweep shared by both stages.  prim: LDS tile [NEQ][NC].  F: x-faces
 // fi=0..16 on rows 1..16 at [k][(j-1)*17+fi]; G: y-faces fj=0..16 on columns
 // 1..16 at [k][fj*16+(i-1)].  choice 2 reconstructs with the limiter.
-// SOLVER / LIM fix the solver and limiter at compile time (-1 / -99: read
+// f0: the thread's first face.  SOLVER / LIM fix the solver and limiter at compile time (-1 / -99: read
 // from p); the arithmetic is the same either way.
 template <int NEQ, int CHOICE, int SOLVER = -1, int LIM = -99>
-__device__ __forceinline__ int flux_sweep_t(const wx_params *__restrict__ p, const double *prim,
+__device__ __forceinline__ int flux_sweep_t(const wx_params *__restrict__ p, int f0, const double *prim,
                                             double *F, double *G) {
   int err = 0;
   const int lim = LIM != -99 ? LIM : p->limiter;
-  for (int f = threadIdx.x; f < 544; f += blockDim.x) {
+  for (int f = f0; f < 544; f += blockDim.x) {
     // x-face fi on row j, or y-face fj on column i: the cells across the face
     // are `stride` apart, and a y-face's states are swapped into the x frame
     // (swapy, src/swapy.f90:4-13), so one solver call serves both
@@ -206,45 +219,138 @@ __device__ __forceinline__ int flux_sweep_t(const wx_params *__restrict__ p, con
 // The sweep with the common configurations compiled in: HLLC, and in
 // stage B the minmod or van Leer limiter; anything else reads p.
 template <int NEQ, int CHOICE>
-__device__ __forceinline__ int flux_sweep(const wx_params *__restrict__ p, const double *prim,
+__device__ __forceinline__ int flux_sweep(const wx_params *__restrict__ p, int f0, const double *prim,
                                           double *F, double *G) {
   if (p->solver == 0) {
-    if (CHOICE == 1) return flux_sweep_t<NEQ, CHOICE, 0>(p, prim, F, G);
-    if (p->limiter == 1) return flux_sweep_t<NEQ, CHOICE, 0, 1>(p, prim, F, G);
-    if (p->limiter == 2) return flux_sweep_t<NEQ, CHOICE, 0, 2>(p, prim, F, G);
+    if (CHOICE == 1) return flux_sweep_t<NEQ, CHOICE, 0>(p, f0, prim, F, G);
+    if (p->limiter == 1) return flux_sweep_t<NEQ, CHOICE, 0, 1>(p, f0, prim, F, G);
+    if (p->limiter == 2) return flux_sweep_t<NEQ, CHOICE, 0, 2>(p, f0, prim, F, G);
   }
-  return flux_sweep_t<NEQ, CHOICE>(p, prim, F, G);
+  return flux_sweep_t<NEQ, CHOICE>(p, f0, prim, F, G);
+}
+
+// The sweep of a block of mild primitives (wx_physics.h).  cs: the cells'
+// sound speeds in the tile's layout (choice 1, whose face states are cells).
+// Returns whether every face of this thread was served.
+template <int NEQ, int CHOICE, int BS, int SOLVER, int LIM>
+__device__ __forceinline__ bool flux_sweep_short(const wx_params *__restrict__ p, int wave, const double *prim,
+                                                 const double *cs, double *F, double *G) {
+  bool ok = true;
+  for (int f = tid_again(wave); f < 544; f += BS) {
+    const bool yf = f >= 272;
+    const int g = yf ? f - 272 : f;
+    const int c0 = yf ? IDX(g % 16 + 1, g / 16) : IDX(g % 17, g / 17 + 1), stride = yf ? NP : 1;
+    double ql[NEQ], qr[NEQ], ff[NEQ];
+#pragma unroll
+    for (int k = 0; k < NEQ; ++k) {
+      const int kk = (k == 1 || k == 2) && yf ? 3 - k : k;
+      ql[k] = prim[kk * NC + c0];
+      qr[k] = prim[kk * NC + c0 + stride];
+    }
+    if constexpr (CHOICE == 2) {
+      double qll[NEQ], qrr[NEQ];
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) {
+        const int kk = (k == 1 || k == 2) && yf ? 3 - k : k;
+        qll[k] = prim[kk * NC + c0 - stride];
+        qrr[k] = prim[kk * NC + c0 + 2 * stride];
+      }
+      limiter_mild<NEQ, LIM>(qll, ql, qr, qrr);
+      const Rcp rl = rdiv(ql[0]), rr = rdiv(qr[0]);
+      const double csl = fsqrt(quot(p->gamma * ql[3], rl)), csr = fsqrt(quot(p->gamma * qr[3], rr));
+      ok = riemann_mild<NEQ, SOLVER, true>(p, ql, qr, csl, csr, rl, rr, ff) & ok;
+    } else {
+      const Rcp none{0.0, 0.0};
+      ok = riemann_mild<NEQ, SOLVER, false>(p, ql, qr, cs[c0], cs[c0 + stride], none, none, ff) & ok;
+    }
+    double *o = yf ? G : F;   // at (j-1)*17+fi and fj*16+(i-1)
+#pragma unroll
+    for (int k = 0; k < NEQ; ++k) {
+      const int kk = (k == 1 || k == 2) && yf ? 3 - k : k;
+      o[kk * 272 + g] = ff[k];
+    }
+  }
+  return ok;
+}
+
+// The short form where it holds (every primitive the faces read is mild; the
+// limiter minmod or van Leer), redone in the general form by the waves that
+// meet a face it does not serve.
+template <int NEQ, int CHOICE, int BS>
+__device__ __forceinline__ int flux_sweep_mild(const wx_params *__restrict__ p, int wave, bool mild, const double *prim,
+                                               const double *cs, double *F, double *G) {
+  bool ok = false;
+  const int solver = p->solver, lim = CHOICE == 1 ? 1 : p->limiter;
+  if (!WX_RARE(!mild) && lim == 1) {
+    if (solver == 0) ok = flux_sweep_short<NEQ, CHOICE, BS, 0, 1>(p, wave, prim, cs, F, G);
+    else if (solver == 1) ok = flux_sweep_short<NEQ, CHOICE, BS, 1, 1>(p, wave, prim, cs, F, G);
+    else ok = flux_sweep_short<NEQ, CHOICE, BS, 2, 1>(p, wave, prim, cs, F, G);
+  } else if (CHOICE == 2 && !WX_RARE(!mild) && lim == 2) {
+    if (solver == 0) ok = flux_sweep_short<NEQ, CHOICE, BS, 0, 2>(p, wave, prim, cs, F, G);
+    else if (solver == 1) ok = flux_sweep_short<NEQ, CHOICE, BS, 1, 2>(p, wave, prim, cs, F, G);
+    else ok = flux_sweep_short<NEQ, CHOICE, BS, 2, 2>(p, wave, prim, cs, F, G);
+  }
+  if (!WX_RARE(!__all(ok))) return 0;
+  return flux_sweep_t<NEQ, CHOICE>(p, tid_again(wave), prim, F, G);
+}
+
+// Whether every wave of the workgroup found its cells mild: each wave's
+// verdict goes to its word of w before a barrier, and is read after it.
+__device__ __forceinline__ void mild_vote(uint32_t *w, int wave, bool ok) {
+  w[wave] = __all(ok) ? 0u : 1u;   // the same word from every lane
+}
+template <int BS>
+__device__ __forceinline__ bool mild_result(const uint32_t *w) {
+  uint32_t bad = 0;
+#pragma unroll
+  for (int k = 0; k < BS / 64; ++k) bad |= w[k];
+  return __builtin_amdgcn_readfirstlane(bad) == 0;
+}
+
+// dt/dx and dt/dy of a block's update (uniform).
+__device__ __forceinline__ void dt_over_dx(const wx_params *__restrict__ p, bool pok, double dt, int level,
+                                           double &dtdx, double &dtdy) {
+  const double dx = p->dx[level - 1], dy = p->dy[level - 1];
+  if (pok && unit_range(dt)) {
+    dtdx = fdiv(dt, dx);
+    dtdy = __double_as_longlong(dx) == __double_as_longlong(dy) ? dtdx : fdiv(dt, dy);
+  } else {
+    dtdx = dt / dx;
+    dtdy = dt / dy;
+  }
 }
 
 // Cylindrical source terms, src/step.f90:49-76 (prims of the stage).
-template <int NEQ>
+template <int NEQ, bool MILD>
 __device__ __forceinline__ void cyl_source(const wx_params *__restrict__ p, const double *prim, int i,
                                            int j, int icy, int lev, double *S) {
   double radius = ((double)(j + icy) - 0.5) * p->dy[lev - 1];
   double rho = prim[0 * NC + IDX(i, j)];
   double v1 = prim[1 * NC + IDX(i, j)], v2 = prim[2 * NC + IDX(i, j)], pr = prim[3 * NC + IDX(i, j)];
   double H = 0.5 * rho * (v1 * v1 + v2 * v2) + (p->cv + 1.) * pr;
-  S[0] = -(rho * v2 / radius);
-  S[1] = -(rho * v1 * v2 / radius);
-  S[2] = -(rho * v2 * v2 / radius);
-  S[3] = -(H * v2 / radius);
+  const Rcp rr = rdiv_<MILD>(radius);
+  S[0] = -quot_<MILD>(rho * v2, rr);
+  S[1] = -quot_<MILD>(rho * v1 * v2, rr);
+  S[2] = -quot_<MILD>(rho * v2 * v2, rr);
+  S[3] = -quot_<MILD>(H * v2, rr);
 #pragma unroll
-  for (int k = 4; k < NEQ; ++k) S[k] = -(prim[k * NC + IDX(i, j)] * v2 / radius);
+  for (int k = 4; k < NEQ; ++k) S[k] = -quot_<MILD>(prim[k * NC + IDX(i, j)] * v2, rr);
 }
 
 // ---------------------------------------------------------------------
 // Stage A: src/tstep.f90:22-46 (hllcfluxes choice 1 + step with dt/2).
-// The one-entry-per-workgroup form is compiled for 8 waves per SIMD (at 512
-// threads that caps it at 64 VGPRs, with a few spills: 8.5 vs 9.2 ns per
-// block at 74 VGPRs and 6 waves on the 16-variant cooling jet; the smaller
-// workgroups are held to fewer waves by their LDS anyway).
-template <int NEQ, int BS, bool PERSIST>
-__global__ __launch_bounds__(BS, PERSIST ? 1 : 8) void k_stageA(const wx_params *__restrict__ P, QueueRef q,
-                                                const double *__restrict__ U, double *__restrict__ Q,
-                                                const double *__restrict__ Pc, DevScalars *__restrict__ Sa) {
+// MILD: the short divisions where they hold (wx_physics.h), and the cells'
+// sound speeds taken once per cell instead of once per face and side.
+template <int NEQ, int BS, bool PERSIST, bool MILD>
+__device__ __forceinline__ void stageA_body(const wx_params *__restrict__ P, QueueRef q, const double *__restrict__ U,
+                                            double *__restrict__ Q, const double *__restrict__ Pc,
+                                            DevScalars *__restrict__ Sa) {
   __shared__ double prim[NEQ * NC];
   __shared__ double F[NEQ * 272];
   __shared__ double G[NEQ * 272];
+  __shared__ double cst[MILD ? 18 * NP : 1];   // sound speeds of rows 0..17
+  __shared__ uint32_t votes[BS / 64];
+  const int wave = wave_of();
   // the first entry's record is read together with the queue length
   const int b0 = PERSIST ? (int)blockIdx.x : xcd_entry(blockIdx.x, gridDim.x);
   LeafRec Lnext = q.rec[min(b0, q.cap - 1)];
@@ -263,34 +369,73 @@ __global__ __launch_bounds__(BS, PERSIST ? 1 : 8) void k_stageA(const wx_params 
   // src/tstep.f90:27-36), not the one u gives back.
   const bool carried = Pc && p->cooling == 2;
   const double *pcb = carried ? Pc + (size_t)L.id * NC : nullptr;
-  for (int c = threadIdx.x; c < 320; c += blockDim.x) {
-    double uu[NEQ], q[NEQ], T;
+  const bool pok = MILD && mild_params(p, L.level);
+  bool ok = pok;
+  if constexpr (MILD) {
+    const RecipP rp = recip_params(p);
+    const double tiny = mild_tiny(p);
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) uu[k] = ub[k * NC + c];
-    uprim<NEQ>(p, q, uu, T);
-    if (carried) q[3] = pcb[c];
-    int i, j;
-    tile_ij(c, i, j);
+    for (int n = 0; n < (320 + BS - 1) / BS; ++n) {
+      const int c = tid_again(wave) + n * BS;
+      if (c >= 320) break;
+      double uu[NEQ], q[NEQ], T;
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(i, j)] = q[k];
+      for (int k = 0; k < NEQ; ++k) uu[k] = ub[k * NC + c];
+      bool okc = uprim_mild<NEQ>(p, rp, tiny, q, uu, T) & pok;
+      if (carried) {
+        q[3] = pcb[c];
+        okc &= (q[3] >= 0x1p-64) & (q[3] <= kHuge);
+      }
+      int i, j;
+      tile_ij(c, i, j);
+      cst[IDX(i, j) - NP] = fsqrt(fdiv(p->gamma * q[3], q[0]));
+      if (WX_RARE(!okc)) {
+        const double pc = q[3];
+        uprim<NEQ>(p, q, uu, T);
+        if (carried) q[3] = pc;
+      }
+      ok &= okc;
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(i, j)] = q[k];
+    }
+    mild_vote(votes, wave, ok);
+  } else {
+    for (int c = tid_again(wave); c < 320; c += BS) {
+      double uu[NEQ], q[NEQ], T;
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) uu[k] = ub[k * NC + c];
+      uprim<NEQ>(p, q, uu, T);
+      if (carried) q[3] = pcb[c];
+      int i, j;
+      tile_ij(c, i, j);
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(i, j)] = q[k];
+    }
   }
   __syncthreads();
-  int err = flux_sweep<NEQ, 1>(p, prim, F, G);
+  const bool mild = MILD && mild_result<BS>(votes);
+  int err;
+  if constexpr (MILD) err = flux_sweep_mild<NEQ, 1, BS>(p, wave, mild, prim, cst - NP, F, G);
+  else err = flux_sweep<NEQ, 1>(p, tid_again(wave), prim, F, G);
   __syncthreads();
-  if (threadIdx.x < 256) {   // one thread per interior cell
+  const int tid = tid_again(wave);
+  if (tid < 256) {   // one thread per interior cell
     const double dtm = S->dt / 2.;
-    const double dtdx = dtm / p->dx[L.level - 1];
-    const double dtdy = dtm / p->dy[L.level - 1];
-    const int i = threadIdx.x % 16 + 1, j = threadIdx.x / 16 + 1;
+    double dtdx, dtdy;
+    dt_over_dx(p, pok, dtm, L.level, dtdx, dtdy);
+    const int i = tid % 16 + 1, j = tid / 16 + 1;
     double Sc[NEQ];
-    if (p->cylindrical) cyl_source<NEQ>(p, prim, i, j, L.icy, L.level, Sc);
+    if (p->cylindrical) {
+      if (mild) cyl_source<NEQ, true>(p, prim, i, j, L.icy, L.level, Sc);
+      else cyl_source<NEQ, false>(p, prim, i, j, L.icy, L.level, Sc);
+    }
     double *qb = Q + (size_t)L.id * NEQ * NC;
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) {
-      double v = ub[k * NC + threadIdx.x] - dtdx * (F[k * 272 + (j - 1) * 17 + i] - F[k * 272 + (j - 1) * 17 + i - 1])
+      double v = ub[k * NC + tid] - dtdx * (F[k * 272 + (j - 1) * 17 + i] - F[k * 272 + (j - 1) * 17 + i - 1])
                  - dtdy * (G[k * 272 + j * 16 + (i - 1)] - G[k * 272 + (j - 1) * 16 + (i - 1)]);
       if (p->cylindrical) v = v + dtm * Sc[k];
-      qb[k * NC + threadIdx.x] = v;
+      qb[k * NC + tid] = v;
     }
   }
   if (err) atomicOr(&S->err, WX_EHLLC);
@@ -299,17 +444,36 @@ __global__ __launch_bounds__(BS, PERSIST ? 1 : 8) void k_stageA(const wx_params 
   }
 }
 
+// The one-entry-per-workgroup form is compiled for 8 waves per SIMD (at 512
+// threads that caps it at 64 VGPRs, with a few spills: 8.5 vs 9.2 ns per
+// block at 74 VGPRs and 6 waves on the 16-variant cooling jet; the smaller
+// workgroups are held to fewer waves by their LDS anyway).
+template <int NEQ, int BS, bool PERSIST>
+__global__ __launch_bounds__(BS, PERSIST ? 1 : 8) void k_stageA(const wx_params *__restrict__ P, QueueRef q,
+                                                const double *__restrict__ U, double *__restrict__ Q,
+                                                const double *__restrict__ Pc, DevScalars *__restrict__ Sa) {
+  stageA_body<NEQ, BS, PERSIST, false>(P, q, U, Q, Pc, Sa);
+}
+template <int NEQ, int BS>
+__global__ __launch_bounds__(BS, 8) void k_stageA_mild(const wx_params *__restrict__ P, QueueRef q,
+                                                const double *__restrict__ U, double *__restrict__ Q,
+                                                const double *__restrict__ Pc, DevScalars *__restrict__ Sa) {
+  stageA_body<NEQ, BS, false, true>(P, q, U, Q, Pc, Sa);
+}
+
 // ---------------------------------------------------------------------
 // Stage B: src/tstep.f90:53-88 with boundaryII pulled from the neighbours.
-template <int NEQ, int BS, bool PERSIST>
-__global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, QueueRef q,
-                                                const int2 *__restrict__ ops,
-                                                const BlockRec *__restrict__ binfo,
-                                                double *__restrict__ U, const double *__restrict__ Q,
-                                                double *__restrict__ Qring, DevScalars *__restrict__ Sa) {
+// MILD: the short divisions where they hold (wx_physics.h).
+template <int NEQ, int BS, bool PERSIST, bool MILD>
+__device__ __forceinline__ void stageB_body(const wx_params *__restrict__ P, QueueRef q, const int2 *__restrict__ ops,
+                                            const BlockRec *__restrict__ binfo, double *__restrict__ U,
+                                            const double *__restrict__ Q, double *__restrict__ Qring,
+                                            DevScalars *__restrict__ Sa) {
   __shared__ double prim[NEQ * NC];
   __shared__ double F[NEQ * 272];
   __shared__ double G[NEQ * 272];
+  __shared__ uint32_t votes[BS / 64];
+  const int wave = wave_of();
   const int b0 = PERSIST ? (int)blockIdx.x : xcd_entry(blockIdx.x, gridDim.x);
   LeafRec Lnext = q.rec[min(b0, q.cap - 1)];
   const int nleaf = q.hdr->nleaf;
@@ -342,14 +506,27 @@ __global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, 
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) u0[k] = ub[k * NC + tid];
   }
+  const bool pok = MILD && mild_params(p, L.level);
+  RecipP rp{};
+  double tiny = 0.0;
+  if constexpr (MILD) {
+    rp = recip_params(p);
+    tiny = mild_tiny(p);
+  }
+  bool ok = true;
+  auto recover = [&](double *q, const double *uu) __attribute__((always_inline)) {
+    double T;
+    if constexpr (MILD) ok &= uprim_any<NEQ>(p, rp, pok, tiny, q, uu, T);
+    else uprim<NEQ>(p, q, uu, T);
+  };
   // interior of U^{n+1/2} (imposed when the block is in the source list)
   if (tid < 256) {
     const int i = tid % 16 + 1, j = tid / 16 + 1;
-    double uu[NEQ], q[NEQ], T;
+    double uu[NEQ], q[NEQ];
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) uu[k] = qb[k * NC + tid];
     if (imp && in_jet(p, L.level, L.icx, L.icy, i, j)) jet_state<NEQ>(p, vjet, uu);
-    uprim<NEQ>(p, q, uu, T);
+    recover(q, uu);
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(i, j)] = q[k];
   }
@@ -358,17 +535,24 @@ __global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, 
   if (ghost) {
     ghost_gather<NEQ>(p, Q, binfo, op, b, L.level, L.icx, L.icy, side, layer, pos, vjet, gh);
     ghost_coords(side, layer, pos, gi, gj);
-    double q[NEQ], T;
-    uprim<NEQ>(p, q, gh, T);
+    double q[NEQ];
+    recover(q, gh);
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(gi, gj)] = q[k];
   }
+  if constexpr (MILD) mild_vote(votes, wave, ok);
   __syncthreads();
-  int err = flux_sweep<NEQ, 2>(p, prim, F, G);
+  const bool mild = MILD && mild_result<BS>(votes);
+  int err;
+  if constexpr (MILD) err = flux_sweep_mild<NEQ, 2, BS>(p, wave, mild, prim, nullptr, F, G);
+  else err = flux_sweep<NEQ, 2>(p, threadIdx.x, prim, F, G);
   __syncthreads();
   const int i = tid % 16 + 1, j = tid / 16 + 1;
   double Sc[NEQ];
-  if (tid < 256 && p->cylindrical) cyl_source<NEQ>(p, prim, i, j, L.icy, L.level, Sc);
+  if (tid < 256 && p->cylindrical) {
+    if (mild) cyl_source<NEQ, true>(p, prim, i, j, L.icy, L.level, Sc);
+    else cyl_source<NEQ, false>(p, prim, i, j, L.icy, L.level, Sc);
+  }
   // the viscosity's stencil (src/viscosity.f90:6-25, on the finest two
   // levels, src/tstep.f90:82) reads Uⁿ of the interior and of ghost layer 1
   // from the primitive tile, which is free after the sweep
@@ -389,8 +573,8 @@ __global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, 
   double un[NEQ];
   if (tid < 256) {   // one thread per interior cell
     const double dt = S->dt;
-    const double dtdx = dt / p->dx[L.level - 1];
-    const double dtdy = dt / p->dy[L.level - 1];
+    double dtdx, dtdy;
+    dt_over_dx(p, pok, dt, L.level, dtdx, dtdy);
     const double eta = p->eta;
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) {
@@ -424,34 +608,38 @@ __global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, 
   }
 }
 
+template <int NEQ, int BS, bool PERSIST>
+__global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, QueueRef q,
+                                                const int2 *__restrict__ ops,
+                                                const BlockRec *__restrict__ binfo,
+                                                double *__restrict__ U, const double *__restrict__ Q,
+                                                double *__restrict__ Qring, DevScalars *__restrict__ Sa) {
+  stageB_body<NEQ, BS, PERSIST, false>(P, q, ops, binfo, U, Q, Qring, Sa);
+}
+template <int NEQ, int BS>
+__global__ __launch_bounds__(BS) void k_stageB_mild(const wx_params *__restrict__ P, QueueRef q,
+                                                const int2 *__restrict__ ops,
+                                                const BlockRec *__restrict__ binfo,
+                                                double *__restrict__ U, const double *__restrict__ Q,
+                                                double *__restrict__ Qring, DevScalars *__restrict__ Sa) {
+  stageB_body<NEQ, BS, false, true>(P, q, ops, binfo, U, Q, Qring, Sa);
+}
+
 // ---------------------------------------------------------------------
 // Block statistics: CFL partials (src/timestep.f90:29-41) and the
 // refinement flag (src/criteria.f90:16-50) from a tile of primitives.
 // Indexed by block ID: stat[2id] = min dx/(|u|+cs), dy/(|v|+cs);
 // stat[2id+1] = DMC t_cool min; flag[id]: 1 refine, 2 coarsen, 0 neither.
 template <int NEQ>
-__device__ void block_stats(const wx_params *__restrict__ p, const double *prim, const LeafRec &L,
-                            double *stat, int8_t *flag, const FlagOut &fo) {
+__device__ __forceinline__ void block_stats(const wx_params *__restrict__ p, bool pok, const double *prim, int id, int lev,
+                                            double *stat, int8_t *flag, int8_t *flagq) {
   __shared__ double red[3][16];
   const int tid = threadIdx.x;
   const int i = tid % 16 + 1, j = tid / 16 + 1;
-  const int lev = L.level;
   double dtp = 1.e30, dtc = 1e30, grad = 0.;
   if (tid < 256) {   // one thread per interior cell
     const double rho = prim[0 * NC + IDX(i, j)], vx = prim[1 * NC + IDX(i, j)];
     const double vy = prim[2 * NC + IDX(i, j)], pr = prim[3 * NC + IDX(i, j)];
-    const double cs = sqrt(p->gamma * pr / rho);
-    dtp = dmin(dtp, p->dx[lev - 1] / (fabs(vx) + cs));
-    dtp = dmin(dtp, p->dy[lev - 1] / (fabs(vy) + cs));
-    if (p->cooling == 2) {
-      double T = (pr / rho) * p->Tempsc;
-      if (T > 1e4) {
-        double al = cooldmc(p, T) * (rho * rho);
-        dtc = dmin(dtc, p->cv * pr / al);
-      }
-    }
-    const double am = dmax(1e-15, fabs(pr));
-    const double am2 = dmax(1e-15, fabs(rho));
     const double *P4 = prim + 3 * NC, *P1 = prim;
     // the reference's max of the four quotients |dP|/am is the quotient of
     // the largest |dP| (a correctly rounded division by am > 0 is monotonic),
@@ -460,7 +648,28 @@ __device__ void block_stats(const wx_params *__restrict__ p, const double *prim,
                                 fabs(P4[IDX(i, j + 1)] - pr)), fabs(P4[IDX(i, j - 1)] - pr));
     const double dr = dmax(dmax(dmax(fabs(P1[IDX(i + 1, j)] - rho), fabs(P1[IDX(i - 1, j)] - rho)),
                                 fabs(P1[IDX(i, j + 1)] - rho)), fabs(P1[IDX(i, j - 1)] - rho));
-    grad = dmax(dp / am, dr / am2);
+    // the short divisions where the cell is in their range (the primitives
+    // are floored; a difference is zero or at least an ulp of them)
+    const bool mild = pok & (rho >= 1e-15) & (rho <= kHuge) & (pr >= 0x1p-64) & (pr <= kHuge) & (fabs(vx) <= kHuge) &
+                      (fabs(vy) <= kHuge) & (dp <= 0x1p200) & (dr <= 0x1p200);
+    auto cell = [&](auto short_form) __attribute__((always_inline)) {
+      constexpr bool M = decltype(short_form)::value;
+      const double cs = sqrt_<M>(div_<M>(p->gamma * pr, rho));
+      dtp = dmin(dtp, div_<M>(p->dx[lev - 1], fabs(vx) + cs));
+      dtp = dmin(dtp, div_<M>(p->dy[lev - 1], fabs(vy) + cs));
+      const double am = dmax(1e-15, fabs(pr));
+      const double am2 = dmax(1e-15, fabs(rho));
+      grad = dmax(div_<M>(dp, am), div_<M>(dr, am2));
+    };
+    if (!WX_RARE(!mild)) cell(std::true_type{});
+    else cell(std::false_type{});
+    if (p->cooling == 2) {
+      double T = (pr / rho) * p->Tempsc;
+      if (T > 1e4) {
+        double al = cooldmc(p, T) * (rho * rho);
+        dtc = dmin(dtc, p->cv * pr / al);
+      }
+    }
   }
   for (int o = 32; o > 0; o >>= 1) {
     dtp = dmin(dtp, __shfl_xor(dtp, o));
@@ -476,13 +685,13 @@ __device__ void block_stats(const wx_params *__restrict__ p, const double *prim,
       dtc = dmin(dtc, red[1][k]);
       grad = dmax(grad, red[2][k]);
     }
-    stat[2 * L.id] = dtp;
-    stat[2 * L.id + 1] = dtc;
+    stat[2 * id] = dtp;
+    stat[2 * id + 1] = dtc;
     int8_t fl = 0;
     if (grad >= p->tol) fl = (lev < p->nlevs) ? 1 : 0;
     else if (grad <= p->tol2) fl = 2;
-    flag[L.id] = fl;
-    if (fo.flagq) fo.flagq[fo.inst_off[L.inst] + L.lidx] = fl;
+    flag[id] = fl;
+    if (flagq) *flagq = fl;
   }
 }
 
@@ -650,7 +859,7 @@ __global__ __launch_bounds__(BS, (SUR ? (PERSIST ? 2 : 1024 / BS) : (PERSIST ? 1
   if (PERSIST && l + (int)gridDim.x < nleaf) Lnext = q.rec[l + gridDim.x];
   const wx_params *__restrict__ p = P + L.inst;
   DevScalars *__restrict__ S = Sa + L.inst;
-  const int b = L.id;
+  const int b = L.id, level = L.level, icx = L.icx, icy = L.icy, inst = L.inst, lidx = L.lidx;
   const int tid = threadIdx.x;
   const double time = S->time;
   const bool imp = (L.flags & 1) != 0;
@@ -663,7 +872,7 @@ __global__ __launch_bounds__(BS, (SUR ? (PERSIST ? 2 : 1024 / BS) : (PERSIST ? 1
     double uu[NEQ];
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) uu[k] = ib[k * NC + c];
-    if (imp && in_jet(p, L.level, L.icx, L.icy, i, j)) jet_state<NEQ>(p, vjet, uu);
+    if (imp && in_jet(p, level, icx, icy, i, j)) jet_state<NEQ>(p, vjet, uu);
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(i, j)] = uu[k];
   }
@@ -679,11 +888,11 @@ __global__ __launch_bounds__(BS, (SUR ? (PERSIST ? 2 : 1024 / BS) : (PERSIST ? 1
     ghost_coords(side, 1, pos, gi, gj);
     double g[NEQ];
     if ((op.y & 15) != GK_NONE) {
-      ghost_gather<NEQ>(p, Uin, binfo, op, b, L.level, L.icx, L.icy, side, 1, pos, vjet, g);
+      ghost_gather<NEQ>(p, Uin, binfo, op, b, level, icx, icy, side, 1, pos, vjet, g);
     } else {
 #pragma unroll
       for (int k = 0; k < NEQ; ++k) g[k] = ob[k * NC + 256 + gt];
-      if (imp && in_jet(p, L.level, L.icx, L.icy, gi, gj)) jet_state<NEQ>(p, vjet, g);
+      if (imp && in_jet(p, level, icx, icy, gi, gj)) jet_state<NEQ>(p, vjet, g);
     }
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(gi, gj)] = g[k];
@@ -695,7 +904,7 @@ __global__ __launch_bounds__(BS, (SUR ? (PERSIST ? 2 : 1024 / BS) : (PERSIST ? 1
     for (int g = tid; g < 64; g += blockDim.x) {
       int gi, gj;
       ghost_coords(g >> 4, 2, (g & 15) + 1, gi, gj);
-      if (in_jet(p, L.level, L.icx, L.icy, gi, gj)) {
+      if (in_jet(p, level, icx, icy, gi, gj)) {
         double v[NEQ];
         jet_state<NEQ>(p, vjet, v);
 #pragma unroll
@@ -718,48 +927,96 @@ __global__ __launch_bounds__(BS, (SUR ? (PERSIST ? 2 : 1024 / BS) : (PERSIST ? 1
     }
   }
   const double dts = S->dt * p->tsc;
+  // the short divisions (wx_physics.h) pay where coolingh runs; without n_HI
+  // they gained nothing (DMC ensemble 44.7 against 45.1 us, 16 blocks of the
+  // adiabatic explosion 5.8 against 6.1)
+  constexpr bool SHORT = NEQ >= 5;
+  const bool pok = SHORT && mild_params(p, level);
+  RecipP rp{};
+  if constexpr (SHORT) rp = recip_params(p);
+  double *pcb = Pc ? Pc + (size_t)b * NC : nullptr;
   // cell c of this thread: cooled state to Uout, its primitives to the tile
   // (under DMC with the cooled pressure, carried into the next step,
-  // src/coolingdmc.f90:27-38)
-  auto cool_pass = [&](auto cool) {
-    for (int c = tid; c < 320; c += blockDim.x) {
-      int i, j;
-      tile_ij(c, i, j);
-      double uu[NEQ];
-#pragma unroll
-      for (int k = 0; k < NEQ; ++k) uu[k] = tile[k * NC + IDX(i, j)];
-      const double pcool = cool(uu);
+  // src/coolingdmc.f90:27-38; the primitives' velocities serve the epilogue's
+  // signal speeds only).  cool returns false, the cell unchanged, where its
+  // short form does not hold; those cells take the general one afterwards.
+  // Neither pass is a loop: the compiler moves the constants of the loop's
+  // exponentials and powers out of it, more than the registers hold (115
+  // scalar-register spills and scratch traffic in every wave).
+  auto cool_pass = [&](auto cool, auto cool_any) __attribute__((always_inline)) {
+    auto put = [&](int c, int i, int j, const double *uu, double pcool) __attribute__((always_inline)) {
 #pragma unroll
       for (int k = 0; k < NEQ; ++k) ob[k * NC + c] = uu[k];
       double q[NEQ], T;
-      uprim<NEQ>(p, q, uu, T);
+      if constexpr (SHORT) uprim_any<NEQ>(p, rp, pok, 0.0, q, uu, T);
+      else uprim<NEQ>(p, q, uu, T);
       if (mode == 2) {
         q[3] = pcool;
-        if (Pc) Pc[(size_t)L.id * NC + c] = pcool;
+        if (pcb) pcb[c] = pcool;
       }
 #pragma unroll
       for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(i, j)] = q[k];
+    };
+    uint32_t left = 0;   // bit n: cell tid + n * BS
+#pragma unroll
+    for (int n = 0; n < (320 + BS - 1) / BS; ++n) {
+      const int c = tid + n * BS;
+      if (c >= 320) break;
+      int i, j;
+      tile_ij(c, i, j);
+      double uu[NEQ], pcool = 0.0;
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) uu[k] = tile[k * NC + IDX(i, j)];
+      if (cool(uu, pcool)) put(c, i, j, uu, pcool);
+      else left |= 1u << n;
+    }
+    if (!WX_RARE(__any(left != 0))) return;
+#pragma unroll
+    for (int n = 0; n < (320 + BS - 1) / BS; ++n) {
+      const int c = tid + n * BS;
+      if (!(left >> n & 1)) continue;
+      int i, j;
+      tile_ij(c, i, j);
+      double uu[NEQ], pcool = 0.0;
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) uu[k] = tile[k * NC + IDX(i, j)];
+      cool_any(uu, pcool);
+      put(c, i, j, uu, pcool);
     }
   };
-  // one loop per cooling mode, so that what the compiler hoists out of one
-  // mode's loop (constants of DMC's log10, kept in scratch memory at this
-  // kernel's register budget) is set up only when that mode runs
   if (!done && mode == 1) {
-    cool_pass([&](double *uu) {
-      atomic_h<NEQ>(p, dts, uu);
-      return 0.0;
-    });
+    cool_pass(
+        [&](double *uu, double &) {
+          if constexpr (NEQ >= 5) {
+            double q[NEQ], T;
+            const bool ok = uprim_mild<NEQ>(p, rp, 0.0, q, uu, T) & pok & (uu[0] >= 1e-15);
+            return ok && atomic_mild<NEQ>(p, rp, dts, q, T, uu);
+          }
+          return true;
+        },
+        [&](double *uu, double &) { atomic_h<NEQ>(p, dts, uu); });
   } else if (!done && mode == 2) {
-    cool_pass([&](double *uu) {
-      double pcool;
-      cool_dmc<NEQ>(p, dts, uu, pcool);
-      return pcool;
-    });
+    cool_pass(
+        [&](double *uu, double &pcool) {
+          double q[NEQ], T;
+          if constexpr (SHORT) {
+            if (!(uprim_mild<NEQ>(p, rp, 0.0, q, uu, T) & pok)) return false;
+          } else {
+            uprim<NEQ>(p, q, uu, T);
+          }
+          cool_dmc<NEQ>(p, dts, q, T, uu, pcool);
+          return true;
+        },
+        [&](double *uu, double &pcool) {
+          double q[NEQ], T;
+          uprim<NEQ>(p, q, uu, T);
+          cool_dmc<NEQ>(p, dts, q, T, uu, pcool);
+        });
   } else if (!done) {
-    cool_pass([](double *) { return 0.0; });
+    cool_pass([](double *, double &) { return true; }, [](double *, double &) {});
   }
   __syncthreads();
-  block_stats<NEQ>(p, tile, L, stat, flag, fo);
+  block_stats<NEQ>(p, pok, tile, b, level, stat, flag, fo.flagq ? fo.flagq + fo.inst_off[inst] + lidx : nullptr);
   __syncthreads();   // the next queue entry reuses the LDS tile
    if (!PERSIST) break;   // one entry per workgroup: no loop
   }
@@ -799,7 +1056,7 @@ __global__ __launch_bounds__(256) void k_blockstat(const wx_params *__restrict__
     for (int k = 0; k < NEQ; ++k) tile[k * NC + IDX(i, j)] = q[k];
   }
   __syncthreads();
-  block_stats<NEQ>(p, tile, L, stat, flag, FlagOut{nullptr, nullptr, nullptr, 0});
+  block_stats<NEQ>(p, mild_params(p, L.level), tile, L.id, L.level, stat, flag, nullptr);
 }
 
 // dt = min(cfl*dtp, 0.4*dtcool*Psc/tsc) (src/timestep.f90:50); optionally
@@ -971,11 +1228,7 @@ __global__ __launch_bounds__(512) void k_meshops(const wx_params *__restrict__ P
   }
   if (!stat) return;
   __syncthreads();
-  LeafRec L{};
-  L.id = dst;
-  L.level = op.level;
-  L.inst = op.inst;
-  block_stats<NEQ>(p, d, L, stat, flag, FlagOut{nullptr, nullptr, nullptr, 0});
+  block_stats<NEQ>(p, mild_params(p, op.level), d, dst, op.level, stat, flag, nullptr);
 }
 
 // Layout transposes between the device's tiles and the reference's
@@ -1079,9 +1332,22 @@ int launch_slot_scatter(const SlotOps *src, int n, int2 *ops, int32_t *flag, hip
   if (PV) { constexpr bool PS = true; CALL; }             \
   else { constexpr bool PS = false; CALL; }
 
+// Launches from which stages A and B use the short divisions.  They take a
+// quarter of the instructions out (stage B 1 167 -> 866 per wave), but a block
+// that holds a velocity below the bound (mild_tiny) pays for both forms, and a
+// small launch lasts as long as its slowest block.  us per launch, general /
+// short: stage A at 1 174 blocks 13.9 / 13.0, at 532 7.8 / 8.2, on 19 250
+// 138 / 122; stage B at 532 11.3 / 12.8, at 1 174 21.0 / 22.9, at 5 322
+// 61.9 / 58.9, at 19 250 218 / 204.
+constexpr int kMildA = 1024, kMildB = 3000;
+
 int launch_stageA(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const double *U,
                   double *Q, const double *Pc, DevScalars *S, hipStream_t stream) {
   if (grid <= 0) return WX_OK;
+  if (!persist && grid >= kMildA) {
+    WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageA_mild<N, B>), dim3(grid), dim3(B), 0, stream, P, q, U, Q, Pc, S)));
+    return hip_status();
+  }
   WX_PERSIST_DISPATCH(persist, WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageA<N, B, PS>), dim3(grid), dim3(B), 0, stream, P, q, U, Q, Pc, S))));
   return hip_status();
 }
@@ -1089,6 +1355,10 @@ int launch_stageA(const wx_params *P, int neq, QueueRef q, int grid, int bs, int
 int launch_stageB(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const int2 *ops,
                   const BlockRec *binfo, double *U, double *Q, DevScalars *S, hipStream_t stream) {
   if (grid <= 0) return WX_OK;
+  if (!persist && grid >= kMildB) {
+    WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageB_mild<N, B>), dim3(grid), dim3(B), 0, stream, P, q, ops, binfo, U, Q, Q, S)));
+    return hip_status();
+  }
   WX_PERSIST_DISPATCH(persist, WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageB<N, B, PS>), dim3(grid), dim3(B), 0, stream, P, q, ops, binfo, U, Q, Q, S))));
   return hip_status();
 }

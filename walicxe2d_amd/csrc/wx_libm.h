@@ -157,7 +157,7 @@ WXM_FN double exp_main(double x, double xtail, uint32_t sign_bias, bool with_tai
 WXM_FN double wexp(double x) {
   bool special = false;
   double y = exp_main(x, 0.0, 0, false, special);
-  if (special) y = exp_kernel(x, 0.0, 0, false);
+  if (__builtin_expect(special, 0)) y = exp_kernel(x, 0.0, 0, false);
   return y;
 }
 
@@ -272,7 +272,7 @@ WXM_FN double pow_main(double x, double y, bool &special) {
 WXM_FN double wpow(double x, double y) {
   bool special = false;
   double r = pow_main(x, y, special);
-  if (special) r = wpow_full(x, y);
+  if (__builtin_expect(special, 0)) r = wpow_full(x, y);
   return r;
 }
 
@@ -308,7 +308,7 @@ WXM_FN double wlog_pow(double x, double y, double *lg) {
   const double elo = fmad(y, lo, fmad(y, hi, -ehi));
   double r = exp_main(ehi, elo, 0, true, special);
   *lg = ix == asu(1.0) ? 0.0 : hi;
-  if (special) {
+  if (__builtin_expect(special, 0)) {
     *lg = wlog(x);
     r = wpow_full(x, y);
   }
