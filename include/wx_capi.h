@@ -114,8 +114,9 @@ int wx_locatebounds(wx_ctx *ctx, int32_t *ninternal);
  * from the tree rows changed since the last build, beside the dt reduction
  * and stage A; 0 on the host (the list itself, compiled, then uploaded);
  * 2 on the device with the scan over block IDs spread over many workgroups
- * at any mesh size (the form it takes above 2048 IDs); 3 (default) on the
- * device from 3072 leaves up, else on the host.  All give identical
+ * at any mesh size (the form it takes above 2048 IDs); 3 (default) by size:
+ * on the device from 16384 leaves up, or from 3072 after a change that
+ * rewrote much of the tree, else on the host.  All give identical
  * tables.  A list set by wx_set_bounds is always compiled on the host. */
 int wx_set_builder(wx_ctx *ctx, int32_t on_device);
 /* The current gather tables, for checks: *nleaf leaf records (8 int32 each:

@@ -273,7 +273,7 @@ class Simulation:
     def set_builder(self, on_device):
         """Build the gather ops on the device (True / 1) or on the host
         (False / 0); 2: on the device with the many-workgroup scan at any
-        size; 3 (the default): on the device from 3072 leaves up."""
+        size; 3 (the default): on the device for large meshes."""
         mode = on_device if isinstance(on_device, int) and not isinstance(on_device, bool) else (1 if on_device else 0)
         _check(self.L.wx_set_builder(self.h, mode), "wx_set_builder")
 

@@ -159,7 +159,8 @@ int graph_span(const EnsGroup *e) {
 void slot_diff(EnsGroup *e, int i, bool two) {
   const Mesh &m = e->m[i];
   EnsGroup::SlotShadow &sh = e->shadow[i];
-  if (!sh.valid) {   // nothing known of the device's copy: every leaf goes up
+  const bool known = sh.valid;
+  if (!known) {   // nothing known of the device's copy: every leaf goes up
     sh.ops2.clear();
     sh.ops1.clear();
     sh.flag.clear();
@@ -173,18 +174,22 @@ void slot_diff(EnsGroup *e, int i, bool two) {
   }
   std::vector<int32_t> &ch = e->changed[i];
   ch.clear();
-  for (size_t l = 0; l < m.leaves.size(); ++l) {
+  auto compare = [&](size_t l) {
     const int id = m.leaves[l].id;
-    const int2 *o2 = &m.opsII[l * 8];
+    const int2 *o2 = m.leaf_ops(l), *o1 = m.opsI_same ? o2 : &m.opsI[l * 8];
     int2 *s2 = &sh.ops2[(size_t)id * 8];
     bool diff = sh.flag[id] != m.leaves[l].flags || memcmp(o2, s2, 8 * sizeof(int2)) != 0;
-    if (two) diff = diff || memcmp(&m.opsI[l * 8], &sh.ops1[(size_t)id * 8], 8 * sizeof(int2)) != 0;
-    if (!diff) continue;
+    if (two) diff = diff || memcmp(o1, &sh.ops1[(size_t)id * 8], 8 * sizeof(int2)) != 0;
+    if (!diff) return;
     memcpy(s2, o2, 8 * sizeof(int2));
-    if (two) memcpy(&sh.ops1[(size_t)id * 8], &m.opsI[l * 8], 8 * sizeof(int2));
+    if (two) memcpy(&sh.ops1[(size_t)id * 8], o1, 8 * sizeof(int2));
     sh.flag[id] = m.leaves[l].flags;
     ch.push_back(id);
-  }
+  };
+  if (known && !m.reops_all)   // only these were recomputed
+    for (int id : m.reops) compare((size_t)m.lidx[id]);
+  else
+    for (size_t l = 0; l < m.leaves.size(); ++l) compare(l);
 }
 
 int upload_queue(EnsGroup *e, const std::vector<int> &stale, bool two);
@@ -212,7 +217,7 @@ int ensure_queue(EnsGroup *e) {
 int upload_queue(EnsGroup *e, const std::vector<int> &stale, bool two) {
   e->pool->run((int)stale.size(), [&](int k) {
     const int i = stale[k];
-    e->rcs[i] = refresh_tables(&e->m[i]);
+    e->rcs[i] = update_tables(&e->m[i]);
     if (e->rcs[i]) {
       e->errs[i] = last_error();
       e->shadow[i].valid = false;

@@ -35,6 +35,7 @@ struct wx_ctx : Mesh, Runtime {
   BlockRec *tBinfo = nullptr;
   int32_t tLeafCap = 0;
   std::vector<BlockRec> tBinfoHost;   // what the arena's block records hold (empty: unknown)
+  std::vector<std::pair<size_t, size_t>> tBinfoRuns;   // upload scratch
   DevBuf<double> dStat;
   DevBuf<int8_t> dFlag;
   DevBuf<double> dScratch;
@@ -101,17 +102,19 @@ int arena_fit(wx_ctx *c) {
   return WX_OK;
 }
 
-// The leaf count from which the device builds the ops when the builder is
-// chosen by size: below it the host compiles the list while the device runs
-// the dt reduction and stage A, and that is the faster of the two (full
-// cooling jet, 1144 leaves: 101 us/step with the host list, 107 with the
-// device builder; point explosion, 5236 leaves: 202 and 192; 9939 leaves:
-// 357 and 311).
-constexpr size_t kDeviceBuilderLeaves = 3072;
+// When the device builds the ops if the builder is chosen by size.  The host
+// brings its list up to date from the rows a mesh change wrote, while the
+// device runs the dt reduction and stage A, and that is the faster of the two
+// up to some 16 000 leaves (us/step, host / device: supernova, 544 leaves
+// 61 / 77; jets, 1 177 92 / 108; 5 319 197 / 205; 9 261 309 / 312; 16 426
+// 573 / 575; 25 633 882 / 875).  A change that rewrites a large part of the
+// tree has the host compile all of it, about 60 ns a leaf, of which stage A
+// hides 8: there the device takes over at 3 072.
+constexpr size_t kDeviceBuilderLeaves = 16384, kDeviceBuilderMany = 3072;
 
 bool use_device_builder(const wx_ctx *c) {
   if (c->dev_builder == 0 || c->bounds_external) return false;
-  return c->dev_builder != 3 || c->leaves.size() >= kDeviceBuilderLeaves;
+  return c->dev_builder != 3 || c->leaves.size() >= (c->many_rows ? kDeviceBuilderMany : kDeviceBuilderLeaves);
 }
 
 // Staged copies of the tree rows written since the device copy was last
@@ -166,24 +169,27 @@ int upload_leaves(wx_ctx *c, bool tree) {
   // mesh change alters the records of a few new blocks)
   std::vector<BlockRec> &dev = c->tBinfoHost;
   const BlockRec *bi = c->binfo.data();
-  std::vector<std::pair<size_t, size_t>> runs;   // [first, last) record indices
+  std::vector<std::pair<size_t, size_t>> &runs = c->tBinfoRuns;   // [first, last) record indices
+  runs.clear();
   size_t nchanged = 0;
-  if (dev.size() != nb) {
-    runs.emplace_back(0, nb);
-    nchanged = nb;
+  auto changed = [&](size_t k) {
+    if (k < dev.size() && memcmp(&bi[k], &dev[k], sizeof(BlockRec)) == 0) return;
+    if (!runs.empty() && runs.back().second == k) runs.back().second = k + 1;
+    else runs.emplace_back(k, k + 1);
+    ++nchanged;
+  };
+  if (c->binfo_all || dev.empty() || dev.size() > nb) {
+    for (size_t k = 0; k < nb; ++k) changed(k);
   } else {
-    for (size_t k = 0; k < nb;) {
-      if (memcmp(&bi[k], &dev[k], sizeof(BlockRec)) == 0) { ++k; continue; }
-      size_t e = k + 1;
-      while (e < nb && memcmp(&bi[e], &dev[e], sizeof(BlockRec)) != 0) ++e;
-      runs.emplace_back(k, e);
-      nchanged += e - k;
-      k = e;
-    }
+    std::vector<int32_t> &ids = c->binfoNew;   // holds every ID above the old maximum
+    std::sort(ids.begin(), ids.end());
+    ids.erase(std::unique(ids.begin(), ids.end()), ids.end());
+    for (int32_t id : ids) changed((size_t)id);
   }
   // unknown until the copies are launched: a failure on the way leaves the
   // shadow empty, so the next upload sends every record
-  dev.clear();
+  std::vector<BlockRec> held;
+  held.swap(dev);
   const size_t tb = tree ? tree_bytes(c) : 0;
   if ((rc = stage_begin(c, al256(512 + bl) + runs.size() * 256 + al256(nchanged * sizeof(BlockRec)) + tb))) return rc;
   char *h = stage_take(c, 512 + bl);
@@ -204,7 +210,11 @@ int upload_leaves(wx_ctx *c, bool tree) {
   }
   if (tree && (rc = stage_tree(c))) return rc;
   if ((rc = stage_end(c))) return rc;
-  dev.assign(bi, bi + nb);
+  dev.swap(held);
+  dev.resize(nb);
+  for (const auto &r : runs) std::copy(bi + r.first, bi + r.second, dev.begin() + (ptrdiff_t)r.first);
+  c->binfoNew.clear();
+  c->binfo_all = false;
   if (tree) {   // the device copy of the tree is current once its copies are launched
     for (int id : c->dirtyRows) c->rowDirty[id] = 0;
     c->dirtyRows.clear();
@@ -215,17 +225,17 @@ int upload_leaves(wx_ctx *c, bool tree) {
 
 // Second half: the ops of both fills (fill I's only where they differ from
 // fill II's, which the fill then reads instead), and the leaf records again
-// when the list set imposition flags in them.
+// when a list from the host set imposition flags in them.
 int upload_ops(wx_ctx *c) {
   const size_t nleaf = c->leaves.size();
   const size_t bo = nleaf * 8 * sizeof(int2), bl = nleaf * sizeof(LeafRec);
-  const bool flags = c->p.otherb != 0, two = !c->opsI_same;
+  const bool flags = c->p.otherb != 0 && c->bounds_external, two = !c->opsI_same;
   int rc = stage_begin(c, (two ? 2 : 1) * al256(bo) + (flags ? al256(bl) : 0));
   if (rc) return rc;
   char *h2 = stage_take(c, bo), *h1 = two ? stage_take(c, bo) : nullptr;
   char *hl = flags ? stage_take(c, bl) : nullptr;
   if (!h2 || (two && !h1) || (flags && !hl)) return fail(WX_EARG, "staging %zu bytes", 2 * bo + bl);
-  memcpy(h2, c->opsII.data(), bo);
+  for (size_t l = 0; l < nleaf; ++l) memcpy(h2 + l * 8 * sizeof(int2), c->leaf_ops(l), 8 * sizeof(int2));
   if ((rc = stage_push(c, c->tOpsII, h2, bo))) return rc;
   if (two) {
     memcpy(h1, c->opsI.data(), bo);
@@ -248,7 +258,7 @@ int upload_ops(wx_ctx *c) {
 int tables_leaves(wx_ctx *c) {
   HostTimer ht(c, HID_TABLES);
   c->flags_host = false;   // leaf positions change
-  int rc = compile_leaves(c);
+  int rc = update_leaves(c);
   const bool dev = use_device_builder(c);
   if (!rc) rc = upload_leaves(c, dev);
   if (rc || !dev) return rc;
@@ -277,8 +287,7 @@ int tables_ops(wx_ctx *c) {
     return WX_OK;
   }
   c->tables_on_device = false;
-  if (!c->bounds_external) locatebounds(c);
-  int rc = compile_ops(c);
+  int rc = update_ops(c);
   if (rc) return rc;
   if ((rc = upload_ops(c))) return rc;
   c->tables_valid = true;
@@ -294,6 +303,7 @@ int ensure_tables(wx_ctx *c) {
 // The list length: the host's, or the device builder's (with a wait).
 int list_length(wx_ctx *c, int32_t *n) {
   if (!c->tables_on_device || !c->tables_valid) {
+    if (c->list_stale && !c->bounds_external) locatebounds(c);
     *n = c->ninternal;
     return WX_OK;
   }

@@ -102,25 +102,26 @@ WXL_FN bool fine_pair(const Tr &t, int nbmax, int nbr, int f, int &n1, int &n2) 
 }
 
 // Writer of one ghost segment: source block, kind | offset << GF_OFF_SHIFT,
-// list position; late: an OUTFYB entry, which boundaryI applies to another
-// block (fill I gets nothing from it here).
+// the leaf whose entry it is and the entry's rank within that leaf's (its list
+// position is the leaf's first plus the rank); late: an OUTFYB entry, which
+// boundaryI applies to another block (fill I gets nothing from it here).
 struct Writer {
-  int src, y, e;
+  int src, y, owner, rank;
   bool late;
 };
 
 // The writer of half h of side s of leaf X; returns 0 or an LBE_* code.
-// info[] holds every block's scanned list offset and count; bc is the box
-// boundary kind of side s; outfyb: the compat mode of src/boundaryI.f90:87
-// with an outflow bottom.
+// bc is the box boundary kind of side s; outfyb: the compat mode of
+// src/boundaryI.f90:87 with an outflow bottom.
 template <class Tr>
-WXL_FN int writer(const Tr &t, int nbmax, const LbInfo *info, int bc, bool outfyb, int X, int s, int h, Writer &w) {
+WXL_FN int writer(const Tr &t, int nbmax, int bc, bool outfyb, int X, int s, int h, Writer &w) {
   w.late = false;
   const int nbr = t.lp(X, 4 + s);
   if (nbr == -1) {   // box face (boundaryII.f90:38-141, boundaryI.f90:38-107)
     w.src = X;
     w.y = bc ? GK_BOXREF : GK_BOXOUT;
-    w.e = info[X].off + face_first(t, nbmax, X, s);
+    w.owner = X;
+    w.rank = face_first(t, nbmax, X, s);
     w.late = outfyb && s == 2;
     return 0;
   }
@@ -135,20 +136,23 @@ WXL_FN int writer(const Tr &t, int nbmax, const LbInfo *info, int bc, bool outfy
     if (j < 0) return LBE_FAMILY;
     w.src = C;
     w.y = GK_PROLONG | ((8 * j) << GF_OFF_SHIFT);
-    w.e = info[C].off + face_first(t, nbmax, C, f) + j;
+    w.owner = C;
+    w.rank = face_first(t, nbmax, C, f) + j;
     return 0;
   }
   if (t.leaf(nbr)) {   // same-level leaf: the entry of the lower ID
     w.src = nbr;
     w.y = GK_COPY;
-    w.e = X < nbr ? info[X].off + face_first(t, nbmax, X, s) : info[nbr].off + face_first(t, nbmax, nbr, s ^ 1);
+    w.owner = X < nbr ? X : nbr;
+    w.rank = X < nbr ? face_first(t, nbmax, X, s) : face_first(t, nbmax, nbr, s ^ 1);
     return 0;
   }
   int n1, n2;   // same level with sons: X's own entry for this half
   if (!fine_pair(t, nbmax, nbr, s, n1, n2)) return LBE_POINTER;
   w.src = h ? n2 : n1;
   w.y = GK_RESTRICT;
-  w.e = info[X].off + face_first(t, nbmax, X, s) + h;
+  w.owner = X;
+  w.rank = face_first(t, nbmax, X, s) + h;
   return 0;
 }
 
@@ -164,21 +168,33 @@ WXL_FN int impose(const LbInfo *info, int src, int dst, int e) {
   return y;
 }
 
+// The same flags without list positions, for an op that is entry `rank` of
+// leaf owner (src or dst): the entries of a block are consecutive and follow
+// those of every lower ID.
+template <class Tr>
+WXL_FN int impose_local(const Tr &t, int nbmax, int src, int dst, int owner, int rank) {
+  int y = 0;
+  if (src == owner ? rank > 0 : (src < owner && block_count(t, nbmax, src) > 0)) y |= GF_SRC_IMPOSED;
+  if (dst == owner || (dst > owner && block_count(t, nbmax, dst) > 0)) y |= GF_DST_IMPOSED;
+  return y;
+}
+
 // The ops of side s (both halves) of leaf X for fills II and I (seg = 2 s +
-// h); bc: the box boundary kind of side s.  e1[h]: the list position of
+// h); info[] holds every block's scanned list offset and count; bc: the box boundary kind of side s.  e1[h]: the list position of
 // fill I's writer of half h (-1: none, an OUTFYB entry of X's own).
 template <class Tr>
 WXL_FN int side_ops(const Tr &t, int nbmax, const LbInfo *info, int bc, bool outfyb, bool otherb, int X, int s,
                     int2 *o2, int2 *o1, int *e1) {
   for (int h = 0; h < 2; ++h) {
     Writer w;
-    const int rc = writer(t, nbmax, info, bc, outfyb, X, s, h, w);
+    const int rc = writer(t, nbmax, bc, outfyb, X, s, h, w);
     if (rc) return rc;
     int y = w.y;
-    if (otherb) y |= impose(info, w.src, X, w.e);
+    const int e = info[w.owner].off + w.rank;
+    if (otherb) y |= impose(info, w.src, X, e);
     o2[h] = int2{w.src, y};
     o1[h] = w.late ? int2{0, GK_NONE} : int2{w.src, y};
-    e1[h] = w.late ? -1 : w.e;
+    e1[h] = w.late ? -1 : e;
   }
   return 0;
 }

@@ -41,8 +41,10 @@ void Mesh::init(const wx_params &pp) {
   up.assign((size_t)cap + 1, 0);
   dn.assign((size_t)cap + 1, 0);
   rowDirty.assign((size_t)cap + 1, 0);
+  mark.assign((size_t)cap + 1, 0);
+  newRows.clear();
   dirtyRows.clear();
-  allDirty = true;
+  all_dirty();
   nbmax = nbleafs = ninternal = 0;
   tables_valid = false;
   bounds_external = false;
@@ -99,6 +101,7 @@ void locatebounds(Mesh *c) {
   }
   out.resize(n);
   c->ninternal = (int)(n / 3);
+  c->list_stale = false;
 }
 
 // ---------------------------------------------------------------------
@@ -114,6 +117,7 @@ struct MeshTree {
 // records, from the tree.
 int compile_leaves(Mesh *c) {
   const int cap = c->nbmax;   // IDs above nbmax hold no block
+  c->leaves_ok = false;
   c->lidx.assign((size_t)cap + 1, -1);
   c->binfo.resize((size_t)cap + 1);
   const int32_t *lp = c->lp.data(), *leaf = c->leaf.data(), *ic = c->icoord.data();
@@ -127,11 +131,14 @@ int compile_leaves(Mesh *c) {
   }
   c->leaves.resize((size_t)nleaf);
   LeafRec *rec = c->leaves.data();
-  const bool otherb = c->p.otherb != 0;
+  const bool otherb = c->p.otherb != 0, counts = otherb || lb_outfyb(c->p);
   const MeshTree tree{lp, leaf};
+  if (counts) c->idCnt.resize((size_t)c->cap + 1);
   for (int nb = 1; nb <= cap; ++nb) {
     const int l = lidx[nb];
     if (l < 0) continue;
+    const int cnt = counts ? std::max(lb::block_count(tree, cap, nb), 0) : 0;
+    if (counts) c->idCnt[nb] = (uint8_t)cnt;
     LeafRec r{};
     r.id = nb;
     r.level = bi[nb].level;
@@ -140,10 +147,15 @@ int compile_leaves(Mesh *c) {
     r.lidx = l;
     // impose_user_bc runs on the block in the fills when it makes list
     // entries (compile_ops sets the same flag from the list itself)
-    if (otherb) r.flags = lb::block_count(tree, cap, nb) > 0 ? 1 : 0;
+    if (otherb) r.flags = cnt > 0 ? 1 : 0;
     if (r.level < 1 || r.level > c->p.nlevs) return fail(WX_EARG, "block %d has level %d", nb, r.level);
     rec[l] = r;
   }
+  for (int nb : c->newRows) c->mark[nb] = 0;
+  c->newRows.clear();
+  c->leaves_ok = true;
+  c->ops_ok = c->ops_pending_id = false;
+  c->reops_all = c->binfo_all = true;
   return WX_OK;
 }
 
@@ -273,7 +285,219 @@ int compile_ops(Mesh *c) {
     if ((o2[k].y & 15) == GK_NONE)
       return fail(WX_EARG, "boundaryII: block %d ghost segment %d not covered by the list",
                   c->leaves[k / 8].id, (int)(k % 8));
+  if (c->bounds_external) {
+    c->leaves_ok = false;   // their imposition flags are that list's
+  } else {
+    if (c->idOps.size() < ((size_t)c->cap + 1) * 8) c->idOps.resize(((size_t)c->cap + 1) * 8);
+    for (int l = 0; l < nleaf; ++l) memcpy(&c->idOps[(size_t)c->leaves[l].id * 8], o2 + (size_t)l * 8, 8 * sizeof(int2));
+    c->ops_ok = true;
+  }
   return WX_OK;
+}
+
+// ---------------------------------------------------------------------
+// The tables after a mesh change, from the rows it wrote.  A step of an
+// adaptive run rewrites a dozen rows of a thousand or more; compiling leaves,
+// list and ops anew took longer than the dt reduction and stage A that hide it
+// (a jet of 2 042 leaves and 11 876 IDs, us per change: leaves 29, list 24,
+// ops 79; from the rows 11 and 14, for 104 of the leaves.  On 1 174 leaves the
+// step goes from 101 to 87 us).
+//
+// A leaf's ops are a function of the rows that lb::writer reads, so they stay
+// as they were unless one of those rows was written.  The ops of leaf X read
+// the rows of X, its face neighbours, the neighbours' sons next to X, and its
+// parent's sons; with a jet source the entry counts of X and of its source
+// blocks too, which read those blocks' neighbours.  Taken backwards: the
+// leaves next to, or sons of, a written row, and with a jet source the leaves
+// next to those.
+static bool next_to(Mesh *c, int n) {
+  const int nbmax = c->nbmax;
+  const MeshTree t{c->lp.data(), c->leaf.data()};
+  auto add = [&](int x) {
+    if (!t.leaf(x) || (c->mark[x] & 2)) return;
+    c->mark[x] |= 2;
+    c->reops.push_back(x);
+  };
+  add(n);
+  for (int f = 0; f < 4; ++f) {
+    const int nbr = t.lp(n, 4 + f);
+    if (nbr < 1) continue;
+    if (nbr > nbmax) return false;
+    if (t.leaf(nbr)) {
+      add(nbr);
+    } else if (t.lp(nbr, 0) == t.lp(n, 0)) {
+      int n1, n2;
+      if (!lb::fine_pair(t, nbmax, nbr, f, n1, n2)) continue;
+      add(n1);
+      add(n2);
+    }
+  }
+  if (!t.leaf(n)) {
+    const int s1 = t.lp(n, 2);
+    if (s1 < 1) return true;
+    if (s1 > nbmax) return false;
+    const int s2 = t.lp(s1, 5), s3 = t.lp(s1, 7);
+    if (!lb::valid(s2, nbmax) || !lb::valid(s3, nbmax)) return false;
+    const int s4 = t.lp(s3, 5);
+    if (!lb::valid(s4, nbmax)) return false;
+    add(s1);
+    add(s2);
+    add(s3);
+    add(s4);
+  }
+  return true;
+}
+
+int update_leaves(Mesh *c) {
+  // many rows at once: the full passes read memory in order (a jet of 1 024
+  // blocks, us from the rows / full: 0.10 written rows a leaf 34 / 70, 0.17
+  // 55 / 71, 0.27 81 / 80, 0.42 121 / 89)
+  c->many_rows = c->leaves_ok && c->newRows.size() > c->leaves.size() / 4;
+  if (!c->leaves_ok || c->bounds_external || c->many_rows) return compile_leaves(c);
+  const int nbmax = c->nbmax;
+  const bool otherb = c->p.otherb != 0, counts = otherb || lb_outfyb(c->p), ops = c->ops_ok;
+  c->leaves_ok = c->ops_ok = c->ops_pending_id = false;   // until all is done
+  std::vector<int32_t> &rows = c->newRows;
+  std::sort(rows.begin(), rows.end());
+  c->binfo.resize((size_t)nbmax + 1);
+  c->lidx.resize((size_t)nbmax + 1, -1);
+  c->leavesOld.swap(c->leaves);
+  const std::vector<LeafRec> &old = c->leavesOld;
+  c->leaves.resize(old.size() + rows.size());
+  LeafRec *rec = c->leaves.data();
+  int *lidx = c->lidx.data();
+  int pos = 0;
+  // the old records before the first written row stay where they are
+  size_t k = rows.empty() ? old.size()
+                          : (size_t)(std::lower_bound(old.begin(), old.end(), rows[0],
+                                                      [](const LeafRec &r, int id) { return r.id < id; }) - old.begin());
+  if (k) memcpy((void *)rec, old.data(), k * sizeof(LeafRec));
+  pos = (int)k;
+  auto keep = [&](size_t to) {   // old records up to `to`
+    for (; k < to; ++k) {
+      rec[pos] = old[k];
+      rec[pos].lidx = pos;
+      lidx[old[k].id] = pos++;
+    }
+  };
+  bool bad = false;
+  for (size_t d = 0; d < rows.size(); ++d) {
+    const int nb = rows[d];
+    if (nb > nbmax) { bad = true; break; }
+    size_t to = k;
+    while (to < old.size() && old[to].id < nb) ++to;
+    keep(to);
+    if (k < old.size() && old[k].id == nb) ++k;
+    c->binfo[nb] = BlockRec{c->LP(nb, 1), c->icoord[(size_t)nb * 2], c->icoord[(size_t)nb * 2 + 1], 0};
+    lidx[nb] = -1;
+    if (!c->leaf[nb]) continue;
+    LeafRec r{};
+    r.id = nb;
+    r.level = c->binfo[nb].level;
+    r.icx = c->binfo[nb].icx;
+    r.icy = c->binfo[nb].icy;
+    r.lidx = pos;
+    if (r.level < 1 || r.level > c->p.nlevs) { bad = true; break; }
+    rec[pos] = r;
+    lidx[nb] = pos++;
+  }
+  if (!bad) keep(old.size());
+  c->leaves.resize((size_t)pos);
+  if (!bad && (ops || counts)) {
+    c->reops.clear();
+    for (size_t d = 0; d < rows.size() && !bad; ++d) bad = !next_to(c, rows[d]);
+    const MeshTree tree{c->lp.data(), c->leaf.data()};
+    const size_t n1 = c->reops.size();
+    for (size_t d = 0; counts && d < n1; ++d) {
+      const int x = c->reops[d], cnt = std::max(lb::block_count(tree, nbmax, x), 0);
+      c->idCnt[x] = (uint8_t)cnt;
+      if (otherb) c->leaves[lidx[x]].flags = cnt > 0 ? 1 : 0;
+    }
+    for (size_t d = 0; otherb && ops && d < n1 && !bad; ++d) bad = !next_to(c, c->reops[d]);
+    for (int x : c->reops) c->mark[x] &= 1;
+  }
+  if (bad) return compile_leaves(c);   // it names what is wrong
+  if (!c->binfo_all) c->binfoNew.insert(c->binfoNew.end(), rows.begin(), rows.end());
+  for (int nb : rows) c->mark[nb] = 0;
+  rows.clear();
+  c->leaves_ok = true;
+  c->ops_pending_id = ops;
+  return WX_OK;
+}
+
+// Fill I's ops in the OUTFYB mode, from fill II's: a bottom box entry, at
+// list position e, writes block e + 1 where that block's own bottom entry does
+// not come later, instead of its own block.  The positions follow from the
+// entry counts (every later one shifts when a block makes more).
+static bool outfyb_ops(Mesh *c) {
+  const MeshTree tree{c->lp.data(), c->leaf.data()};
+  const int nbmax = c->nbmax, nleaf = (int)c->leaves.size();
+  std::vector<int> &off = c->segE1, &late = c->segLate;
+  off.resize((size_t)nleaf);
+  late.clear();
+  c->opsI.resize((size_t)nleaf * 8);
+  int2 *o1 = c->opsI.data();
+  int n = 0;
+  for (int l = 0; l < nleaf; ++l) {
+    const int id = c->leaves[l].id;
+    const int2 *o = &c->idOps[(size_t)id * 8];
+    memcpy(o1 + (size_t)l * 8, o, 8 * sizeof(int2));
+    off[l] = n;
+    n += c->idCnt[id];
+    if ((o[4].y & 15) == GK_BOXOUT) {
+      late.push_back(l);
+      o1[(size_t)l * 8 + 4] = o1[(size_t)l * 8 + 5] = int2{0, GK_NONE};
+    }
+  }
+  for (int l : late) {
+    const int e = off[l] + lb::face_first(tree, nbmax, c->leaves[l].id, 2), t = e + 1;
+    if (t > nbmax || c->lidx[t] < 0) continue;
+    for (int h = 0; h < 2; ++h) {
+      lb::Writer w;
+      if (lb::writer(tree, nbmax, 0, true, t, 2, h, w)) return true;
+      if (!w.late && e <= off[c->lidx[w.owner]] + w.rank) continue;
+      const int owner = c->leaves[l].id;   // of entry e; the block it writes is also its source
+      int y = GK_BOXOUT;
+      if (c->p.otherb) y |= lb::impose_local(tree, nbmax, t, t, owner, e - off[l]);
+      o1[(size_t)c->lidx[t] * 8 + 4 + h] = int2{t, y};
+    }
+  }
+  c->opsI_same = late.empty();
+  c->reops_all = true;
+  return false;
+}
+
+int update_ops(Mesh *c) {
+  if (c->ops_pending_id) {
+    c->ops_pending_id = false;
+    const MeshTree tree{c->lp.data(), c->leaf.data()};
+    const int nbmax = c->nbmax;
+    bool bad = false;
+    for (size_t d = 0; d < c->reops.size() && !bad; ++d) {
+      const int x = c->reops[d];
+      int2 *o = &c->idOps[(size_t)x * 8];
+      for (int sh = 0; sh < 8 && !bad; ++sh) {
+        lb::Writer w;
+        bad = lb::writer(tree, nbmax, c->p.bc[sh >> 1], false, x, sh >> 1, sh & 1, w) != 0;
+        if (bad) break;
+        int y = w.y;
+        if (c->p.otherb) y |= lb::impose_local(tree, nbmax, w.src, x, w.owner, w.rank);
+        o[sh] = int2{w.src, y};
+      }
+    }
+    if (!bad) {
+      c->ops_ok = true;
+      c->reops_all = false;
+      c->opsI_same = true;
+      c->list_stale = true;
+      if (lb_outfyb(c->p)) bad = outfyb_ops(c);
+      if (!bad) return WX_OK;
+      c->ops_ok = false;
+    }
+  }
+  if (!c->bounds_external) locatebounds(c);
+  c->reops_all = true;
+  return compile_ops(c);
 }
 
 // ---------------------------------------------------------------------
@@ -384,37 +608,37 @@ static int admesh_tree(Mesh *c, std::vector<uint8_t> &up, std::vector<uint8_t> &
       updatelpup(c, nb, s1, s2, s3, s4, up, dn);
     }
   }
-  // critneighdown, src/critneighdown.f90:14-50: candidates (first sons that
-  // keep their flag) by level, each level in ascending ID order.  The
-  // coarsening below changes neither levels, sibling numbers nor flags, so
-  // the candidates of every level are known before it starts.
+  // critneighdown, src/critneighdown.f90:14-50: a family coarsens when its
+  // four sons are flagged and none has a finer neighbour.  The coarsening
+  // below changes neither levels, sibling numbers nor flags, so the families
+  // of every level (each level in ascending ID order of the first sons) are
+  // known before it starts.
   std::vector<std::vector<int>> &cand = c->admCand;
   cand.resize((size_t)nlevs + 2);
   for (auto &v : cand) v.clear();
   {
     const int32_t *lp = c->lp.data(), *leaf = c->leaf.data();
-    uint8_t *dnp = dn.data();
+    const uint8_t *dnp = dn.data();
     std::vector<int> &dl = dnl;
     if (!std::is_sorted(dl.begin(), dl.end())) std::sort(dl.begin(), dl.end());
-    for (int nb : dl) {
-      if (!dnp[nb]) continue;
+    auto keep = [&](int nb) {
       const int32_t *L = lp + (size_t)nb * 8;
-      bool keep = true;
-      for (int f = 4; f < 8; ++f) {
-        const int n1 = L[f];
-        if (n1 != -1 && !leaf[n1]) keep = false;
-      }
-      if (!keep) dnp[nb] = 0;
-      else if (nb <= nbmaxp1 && L[3] == 1 && L[0] >= 2 && L[0] <= nlevs) cand[L[0]].push_back(nb);
+      for (int f = 4; f < 8; ++f)
+        if (L[f] != -1 && !leaf[L[f]]) return false;
+      return true;
+    };
+    for (int nb : dl) {
+      const int32_t *L = lp + (size_t)nb * 8;
+      if (!dnp[nb] || nb > nbmaxp1 || L[3] != 1 || L[0] > nlevs || !keep(nb)) continue;
+      const int s2 = L[5], s3 = L[7], s4 = c->LP(s2, 8);
+      if (dnp[s2] && dnp[s3] && dnp[s4] && keep(s2) && keep(s3) && keep(s4)) cand[L[0]].push_back(nb);
     }
   }
   for (int nl = nlevs; nl >= 2; --nl)                // coarsen by level, src/admesh.f90:75-105
     for (int nb : cand[nl]) {
       const int dad = c->LP(nb, 2), s1 = nb, s2 = c->LP(nb, 6), s3 = c->LP(nb, 8), s4 = c->LP(c->LP(nb, 6), 8);
-      if (dn[s2] && dn[s3] && dn[s4]) {
-        ops.push_back(MeshOp{1, dad, s1, s2, s3, s4, 0, 0});
-        updatelpdown(c, dad, s1, s2, s3, s4);
-      }
+      ops.push_back(MeshOp{1, dad, s1, s2, s3, s4, 0, 0});
+      updatelpdown(c, dad, s1, s2, s3, s4);
     }
   // leave the scratch flags cleared for the next call
   for (int nl = 0; nl <= nlevs; ++nl)
@@ -443,12 +667,23 @@ int compile_tables(Mesh *c) {
   return rc ? rc : compile_ops(c);
 }
 
-int refresh_tables(Mesh *c) {
+int update_tables(Mesh *c) {
   if (c->tables_valid) return WX_OK;
-  if (!c->bounds_external) locatebounds(c);
-  int rc = compile_tables(c);
+  int rc = update_leaves(c);
+  if (!rc) rc = update_ops(c);
   if (rc) return rc;
   c->tables_valid = true;
+  return WX_OK;
+}
+
+int refresh_tables(Mesh *c) {
+  int rc = update_tables(c);
+  if (rc || !c->list_stale) return rc;
+  locatebounds(c);
+  const size_t nleaf = c->leaves.size();
+  c->opsII.resize(nleaf * 8);
+  for (size_t l = 0; l < nleaf; ++l) memcpy(&c->opsII[l * 8], c->leaf_ops(l), 8 * sizeof(int2));
+  if (c->opsI_same) c->opsI = c->opsII;
   return WX_OK;
 }
 
@@ -460,7 +695,7 @@ int admesh_from_flags(Mesh *c, const int8_t *flag_of_leaf, std::vector<MeshOp> &
   for (size_t l = 0; l < c->leaves.size(); ++l) {   // markref, src/markref.f90:37-44
     const int id = c->leaves[l].id;
     if (flag_of_leaf[l] == 1) { c->up[id] = 1; upl.push_back(id); }
-    else if (flag_of_leaf[l] == 2) { c->dn[id] = 1; dnl.push_back(id); }
+    else if (flag_of_leaf[l] == 2 && c->leaves[l].level >= 2) { c->dn[id] = 1; dnl.push_back(id); }   // a root has no family
   }
   std::vector<MeshOp> mine;
   int rc = admesh_tree(c, c->up, c->dn, mine, upl, dnl);

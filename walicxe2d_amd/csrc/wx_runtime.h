@@ -68,6 +68,7 @@ struct Mesh {
   int nbmax = 0, nbleafs = 0;
   std::vector<int32_t> bounds;   // the ordered ghost list, [e*3 + c]
   std::vector<uint8_t> bndDone;  // locatebounds scratch
+  bool list_stale = false;       // the tables were brought up to date without the list
   int ninternal = 0;
   // gather tables compiled from the list
   std::vector<LeafRec> leaves;
@@ -97,8 +98,29 @@ struct Mesh {
   std::vector<uint8_t> rowDirty;
   bool allDirty = true;
 
+  // Tables kept up to date from the rows a mesh change wrote (update_leaves,
+  // update_ops).  newRows: the rows written since leaves / lidx / binfo were
+  // current (leaves_ok: they are, but for those rows); idOps: fill II's ops by
+  // block ID, current for the leaves while ops_ok, or, while ops_pending_id,
+  // once the leaves in reops are recomputed; reops_all: every leaf was.
+  // binfoNew: the IDs whose block record was rewritten since the caller
+  // emptied it (binfo_all: any may have been).
+  std::vector<int32_t> newRows, reops, binfoNew;
+  std::vector<uint8_t> mark;   // per ID: 1 in newRows, 2 in reops
+  std::vector<LeafRec> leavesOld;
+  std::vector<int2> idOps;
+  std::vector<uint8_t> idCnt;  // list entries of every leaf, where its flag or the OUTFYB mode needs them
+  bool leaves_ok = false, ops_ok = false, ops_pending_id = false, reops_all = true, binfo_all = true;
+  bool many_rows = false;   // the last change wrote too many rows for that
+  // fill II's ops of leaf l, wherever they are current
+  const int2 *leaf_ops(size_t l) const { return ops_ok ? &idOps[(size_t)leaves[l].id * 8] : &opsII[l * 8]; }
+
   int LP(int nb, int k) const { return lp[(size_t)nb * 8 + k - 1]; }
   void touch(int nb) {
+    if (leaves_ok && !(mark[nb] & 1)) {
+      mark[nb] |= 1;
+      newRows.push_back(nb);
+    }
     if (allDirty || rowDirty[nb]) return;
     rowDirty[nb] = 1;
     dirtyRows.push_back(nb);
@@ -111,6 +133,7 @@ struct Mesh {
     for (int nb : dirtyRows) rowDirty[nb] = 0;
     dirtyRows.clear();
     allDirty = true;
+    leaves_ok = ops_ok = ops_pending_id = false;
   }
   void init(const wx_params &pp);
 };
@@ -124,7 +147,14 @@ void locatebounds(Mesh *m);
 int compile_leaves(Mesh *m);
 int compile_ops(Mesh *m);
 int compile_tables(Mesh *m);
-// locatebounds (unless the list is external) + compile_tables when stale.
+// The same tables from those of the last call and the rows a mesh change wrote
+// since, where that is possible, else compile_leaves and locatebounds (unless
+// the list is external) + compile_ops.
+int update_leaves(Mesh *m);
+int update_ops(Mesh *m);
+// update_leaves + update_ops when stale.
+int update_tables(Mesh *m);
+// The same, and the list and both fills' ops by leaf position with them.
 int refresh_tables(Mesh *m);
 // src/admesh.f90:4-111 from per-leaf flags (flag of leaves[l] at flags[l]:
 // 1 refine, 2 coarsen); appends the data ops and records the new leaves.
