@@ -160,73 +160,94 @@ __device__ __forceinline__ void tile_ij(int c, int &i, int &j) {
   }
 }
 
-// Flux sweep shared by both stages.  prim: LDS tile [NEQ][NC].  F: x-faces
-// fi=0..16 on rows 1..16 at [k][(j-1)*17+fi]; G: y-faces fj=0..16 on columns
-// 1..16 at [k][fj*16+(i-1)].  choice 2 reconstructs with the limiter.
-// f0: the thread's first face.  SOLVER / LIM fix the solver and limiter at compile time (-1 / -99: read
-// from p); the arithmetic is the same either way.
-template <int NEQ, int CHOICE, int SOLVER = -1, int LIM = -99>
-__device__ __forceinline__ int flux_sweep_t(const wx_params *__restrict__ p, int f0, const double *prim,
-                                            double *F, double *G) {
+// The states on the two sides of a face: the cells c0 and c0 + stride of the
+// tile (and the next ones for choice 2's reconstruction).  A y-face's states
+// are swapped into the x frame (swapy, src/swapy.f90:4-13), so one solver call
+// serves both.
+template <int NEQ>
+__device__ __forceinline__ void face_state(const double *prim, int c, bool yf, double *q) {
+#pragma unroll
+  for (int k = 0; k < NEQ; ++k) q[k] = prim[((k == 1 || k == 2) && yf ? 3 - k : k) * NC + c];
+}
+
+// A block's faces, shared out over the workgroup; face(yf, c0, stride, ff)
+// gives the flux.  LDSX: x-face fi = 0..16 of row j goes to F at
+// [k][(j-1)*17+fi], y-face fj = 0..16 of column i to G at [k][fj*16+(i-1)].
+// Otherwise a cell's left x-face stays with the cell's thread (fx, threads
+// below 256) and F is not used: the waves take the 288 other faces first (the
+// y-faces, then the right x-faces of row j to G at [k][272+(j-1)]; the lanes
+// past the last repeat it) and the cells' own last, so that these take
+// registers only after the sweep.
+constexpr int NG = 288;   // fluxes per variable in G
+template <int NEQ, int BS, bool LDSX, class Face>
+__device__ __forceinline__ void sweep_faces(int wave, double *F, double *G, double *fx, Face face) {
+  if constexpr (LDSX) {
+    for (int f = tid_again(wave); f < 544; f += BS) {
+      const bool yf = f >= 272;
+      const int g = yf ? f - 272 : f;
+      const int c0 = yf ? IDX(g % 16 + 1, g / 16) : IDX(g % 17, g / 17 + 1);
+      double ff[NEQ];
+      face(yf, c0, yf ? NP : 1, ff);
+      double *o = yf ? G : F;
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) o[((k == 1 || k == 2) && yf ? 3 - k : k) * 272 + g] = ff[k];
+    }
+  } else {
+    for (int r = wave < 4 ? wave * 64 + BS - 256 : wave * 64 - 256; r < NG || wave < 4; r += BS) {
+      const int tid = tid_again(wave);
+      const bool own = r >= NG;
+      const int g = own ? tid : min(r + (tid & 63), NG - 1);   // cell, or place in G
+      const bool yf = !own && g < 272;
+      const int c0 = yf ? IDX(g % 16 + 1, g / 16) : (own ? IDX(g % 16, g / 16 + 1) : IDX(16, g - 271));
+      double ff[NEQ];
+      face(yf, c0, yf ? NP : 1, ff);
+      if (own) {
+#pragma unroll
+        for (int k = 0; k < NEQ; ++k) fx[k] = ff[k];
+        break;
+      }
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) G[((k == 1 || k == 2) && yf ? 3 - k : k) * NG + g] = ff[k];
+    }
+  }
+}
+
+// Flux sweep shared by both stages.  prim: LDS tile [NEQ][NC].  Choice 1
+// (stage A) takes the fluxes through LDS; choice 2 (stage B) reconstructs with
+// the limiter and keeps the cells' left ones.  SOLVER / LIM fix the solver and
+// limiter at compile time (-1 / -99: read from p); the arithmetic is the same
+// either way.
+template <int NEQ, int CHOICE, int BS, int SOLVER = -1, int LIM = -99>
+__device__ __forceinline__ int flux_sweep_t(const wx_params *__restrict__ p, int wave, const double *prim, double *F,
+                                            double *G, double *fx) {
   int err = 0;
   const int lim = LIM != -99 ? LIM : p->limiter;
-  for (int f = f0; f < 544; f += blockDim.x) {
-    // x-face fi on row j, or y-face fj on column i: the cells across the face
-    // are `stride` apart, and a y-face's states are swapped into the x frame
-    // (swapy, src/swapy.f90:4-13), so one solver call serves both
-    const bool yf = f >= 272;
-    int c0, stride;
-    if (!yf) {
-      c0 = IDX(f % 17, f / 17 + 1);
-      stride = 1;
-    } else {
-      const int g = f - 272;
-      c0 = IDX(g % 16 + 1, g / 16);
-      stride = NP;
-    }
-    double ql[NEQ], qr[NEQ], ff[NEQ];
-#pragma unroll
-    for (int k = 0; k < NEQ; ++k) {
-      const int kk = (k == 1 || k == 2) && yf ? 3 - k : k;
-      ql[k] = prim[kk * NC + c0];
-      qr[k] = prim[kk * NC + c0 + stride];
-    }
-    if (CHOICE == 2) {
+  sweep_faces<NEQ, BS, CHOICE == 1>(wave, F, G, fx, [&](bool yf, int c0, int stride, double *ff) __attribute__((always_inline)) {
+    double ql[NEQ], qr[NEQ];
+    face_state<NEQ>(prim, c0, yf, ql);
+    face_state<NEQ>(prim, c0 + stride, yf, qr);
+    if constexpr (CHOICE == 2) {
       double qll[NEQ], qrr[NEQ];
-#pragma unroll
-      for (int k = 0; k < NEQ; ++k) {
-        const int kk = (k == 1 || k == 2) && yf ? 3 - k : k;
-        qll[k] = prim[kk * NC + c0 - stride];
-        qrr[k] = prim[kk * NC + c0 + 2 * stride];
-      }
+      face_state<NEQ>(prim, c0 - stride, yf, qll);
+      face_state<NEQ>(prim, c0 + 2 * stride, yf, qrr);
       limiter<NEQ>(lim, qll, ql, qr, qrr);
     }
     err |= riemann<NEQ, SOLVER>(p, ql, qr, ff);
-    if (!yf) {
-      const int fi = f % 17, j = f / 17 + 1;
-#pragma unroll
-      for (int k = 0; k < NEQ; ++k) F[k * 272 + (j - 1) * 17 + fi] = ff[k];
-    } else {
-      const int g = f - 272;
-      const int i = g % 16 + 1, fj = g / 16;
-#pragma unroll
-      for (int k = 0; k < NEQ; ++k) G[k * 272 + fj * 16 + (i - 1)] = ff[(k == 1 || k == 2) ? 3 - k : k];
-    }
-  }
+  });
   return err;
 }
 
 // The sweep with the common configurations compiled in: HLLC, and in
 // stage B the minmod or van Leer limiter; anything else reads p.
-template <int NEQ, int CHOICE>
-__device__ __forceinline__ int flux_sweep(const wx_params *__restrict__ p, int f0, const double *prim,
-                                          double *F, double *G) {
+template <int NEQ, int CHOICE, int BS>
+__device__ __forceinline__ int flux_sweep(const wx_params *__restrict__ p, int wave, const double *prim, double *F,
+                                          double *G, double *fx) {
   if (p->solver == 0) {
-    if (CHOICE == 1) return flux_sweep_t<NEQ, CHOICE, 0>(p, f0, prim, F, G);
-    if (p->limiter == 1) return flux_sweep_t<NEQ, CHOICE, 0, 1>(p, f0, prim, F, G);
-    if (p->limiter == 2) return flux_sweep_t<NEQ, CHOICE, 0, 2>(p, f0, prim, F, G);
+    if (CHOICE == 1) return flux_sweep_t<NEQ, CHOICE, BS, 0>(p, wave, prim, F, G, fx);
+    if (p->limiter == 1) return flux_sweep_t<NEQ, CHOICE, BS, 0, 1>(p, wave, prim, F, G, fx);
+    if (p->limiter == 2) return flux_sweep_t<NEQ, CHOICE, BS, 0, 2>(p, wave, prim, F, G, fx);
   }
-  return flux_sweep_t<NEQ, CHOICE>(p, f0, prim, F, G);
+  return flux_sweep_t<NEQ, CHOICE, BS>(p, wave, prim, F, G, fx);
 }
 
 // The sweep of a block of mild primitives (wx_physics.h).  cs: the cells'
@@ -234,27 +255,16 @@ __device__ __forceinline__ int flux_sweep(const wx_params *__restrict__ p, int f
 // Returns whether every face of this thread was served.
 template <int NEQ, int CHOICE, int BS, int SOLVER, int LIM>
 __device__ __forceinline__ bool flux_sweep_short(const wx_params *__restrict__ p, int wave, const double *prim,
-                                                 const double *cs, double *F, double *G) {
+                                                 const double *cs, double *F, double *G, double *fx) {
   bool ok = true;
-  for (int f = tid_again(wave); f < 544; f += BS) {
-    const bool yf = f >= 272;
-    const int g = yf ? f - 272 : f;
-    const int c0 = yf ? IDX(g % 16 + 1, g / 16) : IDX(g % 17, g / 17 + 1), stride = yf ? NP : 1;
-    double ql[NEQ], qr[NEQ], ff[NEQ];
-#pragma unroll
-    for (int k = 0; k < NEQ; ++k) {
-      const int kk = (k == 1 || k == 2) && yf ? 3 - k : k;
-      ql[k] = prim[kk * NC + c0];
-      qr[k] = prim[kk * NC + c0 + stride];
-    }
+  sweep_faces<NEQ, BS, CHOICE == 1>(wave, F, G, fx, [&](bool yf, int c0, int stride, double *ff) __attribute__((always_inline)) {
+    double ql[NEQ], qr[NEQ];
+    face_state<NEQ>(prim, c0, yf, ql);
+    face_state<NEQ>(prim, c0 + stride, yf, qr);
     if constexpr (CHOICE == 2) {
       double qll[NEQ], qrr[NEQ];
-#pragma unroll
-      for (int k = 0; k < NEQ; ++k) {
-        const int kk = (k == 1 || k == 2) && yf ? 3 - k : k;
-        qll[k] = prim[kk * NC + c0 - stride];
-        qrr[k] = prim[kk * NC + c0 + 2 * stride];
-      }
+      face_state<NEQ>(prim, c0 - stride, yf, qll);
+      face_state<NEQ>(prim, c0 + 2 * stride, yf, qrr);
       limiter_mild<NEQ, LIM>(qll, ql, qr, qrr);
       const Rcp rl = rdiv(ql[0]), rr = rdiv(qr[0]);
       const double csl = fsqrt(quot(p->gamma * ql[3], rl)), csr = fsqrt(quot(p->gamma * qr[3], rr));
@@ -263,13 +273,7 @@ __device__ __forceinline__ bool flux_sweep_short(const wx_params *__restrict__ p
       const Rcp none{0.0, 0.0};
       ok = riemann_mild<NEQ, SOLVER, false>(p, ql, qr, cs[c0], cs[c0 + stride], none, none, ff) & ok;
     }
-    double *o = yf ? G : F;   // at (j-1)*17+fi and fj*16+(i-1)
-#pragma unroll
-    for (int k = 0; k < NEQ; ++k) {
-      const int kk = (k == 1 || k == 2) && yf ? 3 - k : k;
-      o[kk * 272 + g] = ff[k];
-    }
-  }
+  });
   return ok;
 }
 
@@ -278,20 +282,32 @@ __device__ __forceinline__ bool flux_sweep_short(const wx_params *__restrict__ p
 // meet a face it does not serve.
 template <int NEQ, int CHOICE, int BS>
 __device__ __forceinline__ int flux_sweep_mild(const wx_params *__restrict__ p, int wave, bool mild, const double *prim,
-                                               const double *cs, double *F, double *G) {
+                                               const double *cs, double *F, double *G, double *fx) {
   bool ok = false;
   const int solver = p->solver, lim = CHOICE == 1 ? 1 : p->limiter;
   if (!WX_RARE(!mild) && lim == 1) {
-    if (solver == 0) ok = flux_sweep_short<NEQ, CHOICE, BS, 0, 1>(p, wave, prim, cs, F, G);
-    else if (solver == 1) ok = flux_sweep_short<NEQ, CHOICE, BS, 1, 1>(p, wave, prim, cs, F, G);
-    else ok = flux_sweep_short<NEQ, CHOICE, BS, 2, 1>(p, wave, prim, cs, F, G);
+    if (solver == 0) ok = flux_sweep_short<NEQ, CHOICE, BS, 0, 1>(p, wave, prim, cs, F, G, fx);
+    else if (solver == 1) ok = flux_sweep_short<NEQ, CHOICE, BS, 1, 1>(p, wave, prim, cs, F, G, fx);
+    else ok = flux_sweep_short<NEQ, CHOICE, BS, 2, 1>(p, wave, prim, cs, F, G, fx);
   } else if (CHOICE == 2 && !WX_RARE(!mild) && lim == 2) {
-    if (solver == 0) ok = flux_sweep_short<NEQ, CHOICE, BS, 0, 2>(p, wave, prim, cs, F, G);
-    else if (solver == 1) ok = flux_sweep_short<NEQ, CHOICE, BS, 1, 2>(p, wave, prim, cs, F, G);
-    else ok = flux_sweep_short<NEQ, CHOICE, BS, 2, 2>(p, wave, prim, cs, F, G);
+    if (solver == 0) ok = flux_sweep_short<NEQ, CHOICE, BS, 0, 2>(p, wave, prim, cs, F, G, fx);
+    else if (solver == 1) ok = flux_sweep_short<NEQ, CHOICE, BS, 1, 2>(p, wave, prim, cs, F, G, fx);
+    else ok = flux_sweep_short<NEQ, CHOICE, BS, 2, 2>(p, wave, prim, cs, F, G, fx);
   }
   if (!WX_RARE(!__all(ok))) return 0;
-  return flux_sweep_t<NEQ, CHOICE>(p, tid_again(wave), prim, F, G);
+  return flux_sweep_t<NEQ, CHOICE, BS>(p, wave, prim, F, G, fx);
+}
+
+// The right x-face's flux of cell tid's thread: its right neighbour's left
+// one (the lane above, within the row of 16), or for the last cell of row j
+// the one in G.  Whole waves.
+__device__ __forceinline__ double flux_right(double left, const double *G, int j) {
+  const double edge = G[272 + j - 1];
+  const uint64_t l = (uint64_t)__double_as_longlong(left), e = (uint64_t)__double_as_longlong(edge);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)e, (int)(uint32_t)l, 0x101, 0xf, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)(e >> 32), (int)(uint32_t)(l >> 32), 0x101, 0xf,
+                                                            0xf, false);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
 // Whether every wave of the workgroup found its cells mild: each wave's
@@ -415,8 +431,8 @@ __device__ __forceinline__ void stageA_body(const wx_params *__restrict__ P, Que
   __syncthreads();
   const bool mild = MILD && mild_result<BS>(votes);
   int err;
-  if constexpr (MILD) err = flux_sweep_mild<NEQ, 1, BS>(p, wave, mild, prim, cst - NP, F, G);
-  else err = flux_sweep<NEQ, 1>(p, tid_again(wave), prim, F, G);
+  if constexpr (MILD) err = flux_sweep_mild<NEQ, 1, BS>(p, wave, mild, prim, cst - NP, F, G, nullptr);
+  else err = flux_sweep<NEQ, 1, BS>(p, wave, prim, F, G, nullptr);
   __syncthreads();
   const int tid = tid_again(wave);
   if (tid < 256) {   // one thread per interior cell
@@ -463,15 +479,15 @@ __global__ __launch_bounds__(BS, 8) void k_stageA_mild(const wx_params *__restri
 
 // ---------------------------------------------------------------------
 // Stage B: src/tstep.f90:53-88 with boundaryII pulled from the neighbours.
-// MILD: the short divisions where they hold (wx_physics.h).
+// Bound by memory latency at the occupancy its registers allow (without the
+// fluxes it takes three quarters of the time).  MILD: the short divisions where they hold (wx_physics.h).
 template <int NEQ, int BS, bool PERSIST, bool MILD>
 __device__ __forceinline__ void stageB_body(const wx_params *__restrict__ P, QueueRef q, const int2 *__restrict__ ops,
                                             const BlockRec *__restrict__ binfo, double *__restrict__ U,
                                             const double *__restrict__ Q, double *__restrict__ Qring,
                                             DevScalars *__restrict__ Sa) {
   __shared__ double prim[NEQ * NC];
-  __shared__ double F[NEQ * 272];
-  __shared__ double G[NEQ * 272];
+  __shared__ double G[NEQ * NG];
   __shared__ uint32_t votes[BS / 64];
   const int wave = wave_of();
   const int b0 = PERSIST ? (int)blockIdx.x : xcd_entry(blockIdx.x, gridDim.x);
@@ -489,23 +505,17 @@ __device__ __forceinline__ void stageB_body(const wx_params *__restrict__ P, Que
   const double vjet = p->otherb ? jet_velocity_at(p, S, time) : 0.0;
   const double *qb = Q + (size_t)b * NEQ * NC;
   double *ub = U + (size_t)b * NEQ * NC;
-  const int tid = threadIdx.x;
+  const int tid0 = tid_again(wave);
   // two-layer ghost ring: 4 sides x 2 layers x 16 positions = 128 cells,
   // gathered by waves of their own when the workgroup has them.  The op of
-  // the ghost's segment and Uⁿ of the thread's interior cell (used by the
-  // update after the sweep) are read first, so that their latency overlaps
-  // the interior's primitive recovery.
-  const int gt = BS >= 384 ? tid - 256 : tid;
+  // the ghost's segment is read first, so that its latency overlaps the
+  // interior's primitive recovery.
+  const int gt = BS >= 384 ? tid0 - 256 : tid0;
   const bool ghost = gt >= 0 && gt < 128;
   const int side = gt >> 5, layer = ((gt >> 4) & 1) + 1, pos = (gt & 15) + 1;
   const bool keep1 = (p->compat & 2) && p->bc[2] == 0;   // lb_outfyb
   int2 op = make_int2(0, 0);
   if (ghost) op = ops[r * 8 + side * 2 + ((pos - 1) >> 3)];
-  double u0[NEQ];
-  if (tid < 256) {
-#pragma unroll
-    for (int k = 0; k < NEQ; ++k) u0[k] = ub[k * NC + tid];
-  }
   const bool pok = MILD && mild_params(p, L.level);
   RecipP rp{};
   double tiny = 0.0;
@@ -520,21 +530,31 @@ __device__ __forceinline__ void stageB_body(const wx_params *__restrict__ P, Que
     else uprim<NEQ>(p, q, uu, T);
   };
   // interior of U^{n+1/2} (imposed when the block is in the source list)
-  if (tid < 256) {
-    const int i = tid % 16 + 1, j = tid / 16 + 1;
+  if (tid0 < 256) {
+    const int i = tid0 % 16 + 1, j = tid0 / 16 + 1;
     double uu[NEQ], q[NEQ];
 #pragma unroll
-    for (int k = 0; k < NEQ; ++k) uu[k] = qb[k * NC + tid];
+    for (int k = 0; k < NEQ; ++k) uu[k] = qb[k * NC + tid0];
     if (imp && in_jet(p, L.level, L.icx, L.icy, i, j)) jet_state<NEQ>(p, vjet, uu);
     recover(q, uu);
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) prim[k * NC + IDX(i, j)] = q[k];
   }
-  double gh[NEQ];
-  int gi = 0, gj = 0;
   if (ghost) {
+    double gh[NEQ];
+    int gi, gj;
     ghost_gather<NEQ>(p, Q, binfo, op, b, L.level, L.icx, L.icy, side, layer, pos, vjet, gh);
     ghost_coords(side, layer, pos, gi, gj);
+    // the ring of U^{n+1/2} goes to its own tile's ring in the U^{n+1/2}
+    // buffer (Qring is Q: this launch reads only interiors of Q), where the
+    // fill leaves layer 2 as the step's final value (src/tstep.f90:85 copies
+    // up's ring into u; boundaryI rewrites layer 1, except the segments that
+    // the OUTFYB mode's list leaves to the carried values)
+    if (layer == 2 || keep1) {
+      double *rb = Qring + (size_t)b * NEQ * NC + 256 + (layer - 1) * 64 + side * 16 + pos - 1;
+#pragma unroll
+      for (int k = 0; k < NEQ; ++k) rb[k * NC] = gh[k];
+    }
     double q[NEQ];
     recover(q, gh);
 #pragma unroll
@@ -544,8 +564,15 @@ __device__ __forceinline__ void stageB_body(const wx_params *__restrict__ P, Que
   __syncthreads();
   const bool mild = MILD && mild_result<BS>(votes);
   int err;
-  if constexpr (MILD) err = flux_sweep_mild<NEQ, 2, BS>(p, wave, mild, prim, nullptr, F, G);
-  else err = flux_sweep<NEQ, 2>(p, threadIdx.x, prim, F, G);
+  double fx[NEQ];
+  if constexpr (MILD) err = flux_sweep_mild<NEQ, 2, BS>(p, wave, mild, prim, nullptr, nullptr, G, fx);
+  else err = flux_sweep<NEQ, 2, BS>(p, wave, prim, nullptr, G, fx);
+  const int tid = tid_again(wave);
+  double u0[NEQ];
+  if (tid < 256) {
+#pragma unroll
+    for (int k = 0; k < NEQ; ++k) u0[k] = ub[k * NC + tid];
+  }
   __syncthreads();
   const int i = tid % 16 + 1, j = tid / 16 + 1;
   double Sc[NEQ];
@@ -579,8 +606,8 @@ __device__ __forceinline__ void stageB_body(const wx_params *__restrict__ P, Que
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) {
       const double *uk = prim + k * NC;
-      double v = u0[k] - dtdx * (F[k * 272 + (j - 1) * 17 + i] - F[k * 272 + (j - 1) * 17 + i - 1])
-                 - dtdy * (G[k * 272 + j * 16 + (i - 1)] - G[k * 272 + (j - 1) * 16 + (i - 1)]);
+      double v = u0[k] - dtdx * (flux_right(fx[k], G + k * NG, j) - fx[k])
+                 - dtdy * (G[k * NG + j * 16 + (i - 1)] - G[k * NG + (j - 1) * 16 + (i - 1)]);
       if (p->cylindrical) v = v + dt * Sc[k];
       if (visc)   // no dt factor
         v = v + eta * (uk[IDX(i + 1, j)] + uk[IDX(i - 1, j)] + uk[IDX(i, j + 1)] + uk[IDX(i, j - 1)] - 4. * u0[k]);
@@ -592,24 +619,21 @@ __device__ __forceinline__ void stageB_body(const wx_params *__restrict__ P, Que
   if (tid < 256)
 #pragma unroll
     for (int k = 0; k < NEQ; ++k) ub[k * NC + tid] = un[k];
-  // the ring of U^{n+1/2} goes to its own tile's ring in the U^{n+1/2}
-  // buffer (Qring is Q: this launch reads only interiors of Q), where the
-  // fill leaves layer 2 as the step's final value (src/tstep.f90:85 copies
-  // up's ring into u; boundaryI rewrites layer 1, except the segments that
-  // the OUTFYB mode's list leaves to the carried values)
-  if (ghost && (layer == 2 || keep1)) {
-    double *rb = Qring + (size_t)b * NEQ * NC + 256 + (layer - 1) * 64 + side * 16 + pos - 1;
-#pragma unroll
-    for (int k = 0; k < NEQ; ++k) rb[k * NC] = gh[k];
-  }
   if (err) atomicOr(&S->err, WX_EHLLC);
   __syncthreads();   // the next queue entry reuses the LDS tiles
    if (!PERSIST) break;   // one entry per workgroup: no loop
   }
 }
 
+// Five workgroups on a compute unit: 27.5 KB of LDS (the cells' left x-fluxes
+// stay in registers and cross to the left neighbour between lanes; with all of
+// them in LDS it was 37.8 KB) and 96 VGPRs (the ghosts are written out when
+// gathered, U^n is read after the sweep).  us per launch at four / five:
+// 1 174 blocks, of which four hold 1 024 at a time, 21.6 / 19.6; 5 319
+// 58.5 / 54.3; 19 250 203 / 191.  Six variables need more registers.
+constexpr int kStageBWaves = 5;
 template <int NEQ, int BS, bool PERSIST>
-__global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, QueueRef q,
+__global__ __launch_bounds__(BS, PERSIST || NEQ > 5 ? 1 : kStageBWaves) void k_stageB(const wx_params *__restrict__ P, QueueRef q,
                                                 const int2 *__restrict__ ops,
                                                 const BlockRec *__restrict__ binfo,
                                                 double *__restrict__ U, const double *__restrict__ Q,
@@ -617,7 +641,7 @@ __global__ __launch_bounds__(BS) void k_stageB(const wx_params *__restrict__ P, 
   stageB_body<NEQ, BS, PERSIST, false>(P, q, ops, binfo, U, Q, Qring, Sa);
 }
 template <int NEQ, int BS>
-__global__ __launch_bounds__(BS) void k_stageB_mild(const wx_params *__restrict__ P, QueueRef q,
+__global__ __launch_bounds__(BS, NEQ > 5 ? 1 : kStageBWaves) void k_stageB_mild(const wx_params *__restrict__ P, QueueRef q,
                                                 const int2 *__restrict__ ops,
                                                 const BlockRec *__restrict__ binfo,
                                                 double *__restrict__ U, const double *__restrict__ Q,
@@ -1072,11 +1096,23 @@ __global__ __launch_bounds__(1024) void k_dtreduce(const wx_params *__restrict__
   DevScalars *__restrict__ S = Sa + inst;
   const int n = inst_off[inst + 1] - inst_off[inst];
   const LeafRec *__restrict__ mine = rec + inst_off[inst];
+  // what the last thread needs is read with the first loads of the chain
+  // inst_off -> rec -> stat, not after it
+  const double cfl = p->cfl, Psc = p->Psc, tsc = p->tsc, time = S->time;
+  const bool jet = p->otherb != 0;
   double a = 1.e30, c = 1e30;
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const int id = mine[k].id;
-    a = dmin(a, stat[2 * id]);
-    c = dmin(c, stat[2 * id + 1]);
+  // four records a round: a record's ID and then its partials are two trips to
+  // memory, and one workgroup makes them all (5 319 leaves: 9.5 us one record
+  // at a time, 7.9 now)
+  for (int k = threadIdx.x; k < n; k += 4 * blockDim.x) {
+    int id[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) id[u] = mine[min(k + u * (int)blockDim.x, n - 1)].id;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      a = dmin(a, stat[2 * id[u]]);
+      c = dmin(c, stat[2 * id[u] + 1]);
+    }
   }
   for (int o = 32; o > 0; o >>= 1) {
     a = dmin(a, __shfl_xor(a, o));
@@ -1089,11 +1125,11 @@ __global__ __launch_bounds__(1024) void k_dtreduce(const wx_params *__restrict__
     for (int k = 1; k < nw; ++k) { a = dmin(a, r0[k]); c = dmin(c, r1[k]); }
     S->dtp_min = a;
     S->dtcool_min = c;
-    double dt = dmin(p->cfl * a, 0.4 * c * p->Psc / p->tsc);
+    double dt = dmin(cfl * a, 0.4 * c * Psc / tsc);
     S->dt = dt;
-    if (advance) S->time = S->time + dt;
-    if (p->otherb) {   // the jet source speed of the step, once instead of per wave of the stages
-      const double t = S->time;
+    const double t = advance ? time + dt : time;
+    if (advance) S->time = t;
+    if (jet) {   // the jet source speed of the step, once instead of per wave of the stages
       S->vjet = jet_velocity(p, t);
       S->vjet_time = t;
       S->vjet_ok = 1;
@@ -1337,8 +1373,8 @@ int launch_slot_scatter(const SlotOps *src, int n, int2 *ops, int32_t *flag, hip
 // that holds a velocity below the bound (mild_tiny) pays for both forms, and a
 // small launch lasts as long as its slowest block.  us per launch, general /
 // short: stage A at 1 174 blocks 13.9 / 13.0, at 532 7.8 / 8.2, on 19 250
-// 138 / 122; stage B at 532 11.3 / 12.8, at 1 174 21.0 / 22.9, at 5 322
-// 61.9 / 58.9, at 19 250 218 / 204.
+// 138 / 122; stage B at 520 11.9 / 13.1, at 1 177 19.6 / 20.2, at 5 319
+// 58.4 / 54.2, at 19 250 206 / 191.
 constexpr int kMildA = 1024, kMildB = 3000;
 
 int launch_stageA(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const double *U,
@@ -1422,7 +1458,12 @@ __global__ __launch_bounds__(256) void k_h2d(const CopyDesc *__restrict__ d, int
   if ((al & 15) == 0) {
     const uint4 *s = (const uint4 *)c.src;
     uint4 *o = (uint4 *)c.dst;
-    for (size_t i = t0; i < c.bytes / 16; i += st) o[i] = s[i];
+    const size_t n = c.bytes / 16;
+    for (size_t i = t0; i < n; i += 2 * st) {   // two words in flight: a read crosses the host link
+      const uint4 v = s[i], w = s[i + st < n ? i + st : i];
+      o[i] = v;
+      if (i + st < n) o[i + st] = w;
+    }
   } else if ((al & 3) == 0) {
     const uint32_t *s = (const uint32_t *)c.src;
     uint32_t *o = (uint32_t *)c.dst;
