@@ -377,6 +377,14 @@ int sync_scalars(wx_ctx *c) {
 // Stage A runs in 8-wave workgroups, the others in 4-wave ones: the fastest
 // shapes on the full cooling jet (1162 leaves: stage A 14.4 ns per block at
 // 512 threads, 16.0 at 256; stage B and the fill 2-5 ns slower at 384 or 512).
+// Up to two blocks a compute unit a launch lasts as long as one block, so more
+// threads share it: stage B takes 512, the fill 384 (its 320 cells in one
+// pass).  us/step at 256 threads / so: explosion, 36 blocks 21.3 / 20.1, 484
+// 26.2 / 25.3, 676 30.8 / 32.7; jet, 96 29.3 / 26.2, 512 35.2 / 32.4, 768
+// 41.5 / 46.5; with the hybrid solver, 200 38.4 / 32.6, 512 43.7 / 39.4, 768
+// 54.3 / 60.8.
+constexpr int kFewLeaves = 512;
+
 int run_stage_a(wx_ctx *c) {
   ProfScope ps(c, KID_STAGEA);
   int rc = launch_stageA(c->dP.ptr, c->neq, c->queue(), c->nleaf(), 512, 0, c->cur_u(), c->other_u(), c->pc(),
@@ -387,10 +395,11 @@ int run_stage_a(wx_ctx *c) {
 
 int run_stages_bf(wx_ctx *c) {
   const int g = c->nleaf();   // one workgroup per queue entry
+  const int bsB = g <= kFewLeaves ? 512 : 256, bsF = g <= kFewLeaves ? 384 : 256;
   int rc;
   {
     ProfScope ps(c, KID_STAGEB);
-    rc = launch_stageB(c->dP.ptr, c->neq, c->queue(), g, 256, 0, c->tOpsII, c->tBinfo, c->cur_u(), c->other_u(),
+    rc = launch_stageB(c->dP.ptr, c->neq, c->queue(), g, bsB, 0, c->tOpsII, c->tBinfo, c->cur_u(), c->other_u(),
                        c->dS.ptr, c->stream);
   }
   if (!rc) {
@@ -398,10 +407,10 @@ int run_stages_bf(wx_ctx *c) {
     const FlagOut fo{c->tOff, c->hFlagQ_dev, c->hS_dev, 1};
     const int2 *opsI = c->opsI_same ? c->tOpsII : c->tOpsI;
     if (c->use_sur)
-      rc = launch_fillI_cool_sur(c->dP.ptr, c->neq, c->queue(), g, 256, 0, opsI, c->tBinfo, c->cur_u(),
+      rc = launch_fillI_cool_sur(c->dP.ptr, c->neq, c->queue(), g, bsF, 0, opsI, c->tBinfo, c->cur_u(),
                                  c->other_u(), c->dStat.ptr, c->dFlag.ptr, c->dS.ptr, c->dSur.ptr, fo, c->stream);
     else
-      rc = launch_fillI_cool(c->dP.ptr, c->neq, c->queue(), g, 256, 0, opsI, c->tBinfo, c->cur_u(),
+      rc = launch_fillI_cool(c->dP.ptr, c->neq, c->queue(), g, bsF, 0, opsI, c->tBinfo, c->cur_u(),
                              c->other_u(), c->dStat.ptr, c->dFlag.ptr, c->dS.ptr, fo, c->pc(), c->stream);
   }
   if (rc) return fail(rc, "stage launch failed: %s", hipGetErrorString(hipGetLastError()));
