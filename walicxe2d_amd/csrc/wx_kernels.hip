@@ -654,14 +654,22 @@ __global__ __launch_bounds__(BS, NEQ > 5 ? 1 : kStageBWaves) void k_stageB_mild(
 // refinement flag (src/criteria.f90:16-50) from a tile of primitives.
 // Indexed by block ID: stat[2id] = min dx/(|u|+cs), dy/(|v|+cs);
 // stat[2id+1] = DMC t_cool min; flag[id]: 1 refine, 2 coarsen, 0 neither.
-template <int NEQ>
+// BS below 256: each wave takes several groups of 64 cells, one after the
+// other, and the groups are folded in the same order.
+template <int NEQ, int BS = 256>
 __device__ __forceinline__ void block_stats(const wx_params *__restrict__ p, bool pok, const double *prim, int id, int lev,
                                             double *stat, int8_t *flag, int8_t *flagq) {
   __shared__ double red[3][16];
   const int tid = threadIdx.x;
-  const int i = tid % 16 + 1, j = tid / 16 + 1;
-  double dtp = 1.e30, dtc = 1e30, grad = 0.;
-  if (tid < 256) {   // one thread per interior cell
+  double dtp, dtc, grad;
+#pragma unroll 1
+  for (int n = 0; n < (BS < 256 ? 256 / BS : 1); ++n) {
+  const int cell_id = tid + n * BS;
+  const int i = cell_id % 16 + 1, j = cell_id / 16 + 1;
+  dtp = 1.e30;
+  dtc = 1e30;
+  grad = 0.;
+  if (cell_id < 256) {   // one thread per interior cell
     const double rho = prim[0 * NC + IDX(i, j)], vx = prim[1 * NC + IDX(i, j)];
     const double vy = prim[2 * NC + IDX(i, j)], pr = prim[3 * NC + IDX(i, j)];
     const double *P4 = prim + 3 * NC, *P1 = prim;
@@ -700,11 +708,17 @@ __device__ __forceinline__ void block_stats(const wx_params *__restrict__ p, boo
     dtc = dmin(dtc, __shfl_xor(dtc, o));
     grad = dmax(grad, __shfl_xor(grad, o));
   }
-  const int w = tid >> 6;
+  const int w = cell_id >> 6;
   if ((tid & 63) == 0) { red[0][w] = dtp; red[1][w] = dtc; red[2][w] = grad; }
+  }
   __syncthreads();
   if (tid == 0) {
-    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) {
+    if (BS < 256) {
+      dtp = red[0][0];
+      dtc = red[1][0];
+      grad = red[2][0];
+    }
+    for (int k = 1; k < (BS < 256 ? 4 : (int)(blockDim.x >> 6)); ++k) {
       dtp = dmin(dtp, red[0][k]);
       dtc = dmin(dtc, red[1][k]);
       grad = dmax(grad, red[2][k]);
@@ -1040,7 +1054,7 @@ __global__ __launch_bounds__(BS, (SUR ? (PERSIST ? 2 : 1024 / BS) : (PERSIST ? 1
     cool_pass([](double *, double &) { return true; }, [](double *, double &) {});
   }
   __syncthreads();
-  block_stats<NEQ>(p, pok, tile, b, level, stat, flag, fo.flagq ? fo.flagq + fo.inst_off[inst] + lidx : nullptr);
+  block_stats<NEQ, BS>(p, pok, tile, b, level, stat, flag, fo.flagq ? fo.flagq + fo.inst_off[inst] + lidx : nullptr);
   __syncthreads();   // the next queue entry reuses the LDS tile
    if (!PERSIST) break;   // one entry per workgroup: no loop
   }
@@ -1399,10 +1413,26 @@ int launch_stageB(const wx_params *P, int neq, QueueRef q, int grid, int bs, int
   return hip_status();
 }
 
+// Launches of tiles with n_HI from which the fill takes two waves per block
+// instead of four.  Its 320 cells are five passes of a wave: four waves take
+// two rounds, three of them idle in the second (five of eight slots used), two
+// take three rounds (five of six), and ten such workgroups fill a compute unit
+// to the byte of LDS and at the same five waves per SIMD.  A block takes longer,
+// so it needs many rounds of blocks: passes of 5 322 blocks 80.3 -> 81.6 ms, of
+// ensembles without n_HI 125.5 -> 127.1, of two groups of 9 600 blocks
+// 297.4 -> 293.4.
+constexpr int kFill128 = 8192;
+
 int launch_fillI_cool(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const int2 *ops,
                       const BlockRec *binfo, const double *Uin, double *Uout, double *stat, int8_t *flag,
                       DevScalars *S, FlagOut fo, double *Pc, hipStream_t stream) {
   if (grid <= 0) return WX_OK;
+  if (!persist && bs == 256 && neq >= 5 && grid >= kFill128) {
+    if (neq == 5) hipLaunchKernelGGL((k_fillI_cool<5, false, 128, false>), dim3(grid), dim3(128), 0, stream, P, q, ops, binfo, Uin, Uout, stat, flag, S, fo, nullptr, Pc);
+    else if (neq == 6) hipLaunchKernelGGL((k_fillI_cool<6, false, 128, false>), dim3(grid), dim3(128), 0, stream, P, q, ops, binfo, Uin, Uout, stat, flag, S, fo, nullptr, Pc);
+    else return WX_EARG;
+    return hip_status();
+  }
   WX_PERSIST_DISPATCH(persist, WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_fillI_cool<N, false, B, PS>), dim3(grid), dim3(B), 0, stream, P, q, ops, binfo, Uin, Uout, stat, flag, S, fo, nullptr, Pc))));
   return hip_status();
 }
