@@ -1124,8 +1124,12 @@ __global__ __launch_bounds__(1024) void k_dtreduce(const wx_params *__restrict__
     for (int u = 0; u < 4; ++u) id[u] = mine[min(k + u * (int)blockDim.x, n - 1)].id;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      a = dmin(a, stat[2 * id[u]]);
-      c = dmin(c, stat[2 * id[u] + 1]);
+      // no record twice: a minimum with a NaN takes its other operand or not by
+      // their order
+      const double sa = stat[2 * id[u]], sc = stat[2 * id[u] + 1];
+      const bool in = k + u * (int)blockDim.x < n;
+      a = in ? dmin(a, sa) : a;
+      c = in ? dmin(c, sc) : c;
     }
   }
   for (int o = 32; o > 0; o >>= 1) {
