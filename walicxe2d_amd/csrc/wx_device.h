@@ -75,7 +75,11 @@ struct QueueRef {
   const QueueHdr *hdr;
   const LeafRec *rec;
   int32_t cap;
+  const double *stat;   // set where stage A takes the step's dt from the CFL partials itself
 };
+
+// launch_dtreduce's `advance` where the step's stage A takes dt: nothing to launch.
+constexpr int kDtInStageA = 2;
 
 // Per-ID record for source lookups (level and lower-left cell index).
 struct BlockRec {

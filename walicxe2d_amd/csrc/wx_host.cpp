@@ -383,11 +383,19 @@ int sync_scalars(wx_ctx *c) {
 // 26.2 / 25.3, 676 30.8 / 32.7; jet, 96 29.3 / 26.2, 512 35.2 / 32.4, 768
 // 41.5 / 46.5; with the hybrid solver, 200 38.4 / 32.6, 512 43.7 / 39.4, 768
 // 54.3 / 60.8.
+// Up to there stage A also takes the dt reduction, a launch of one workgroup
+// that costs 4-5 us by itself against about 2 us in stage A (a trip for the
+// leaf records and one for their partials): explosion, 16 blocks, 22.2 / 18.7
+// us per step, jet of about 450 with the hybrid solver 63.9 / 62.3; above, a
+// thread would take several records.
 constexpr int kFewLeaves = 512;
 
-int run_stage_a(wx_ctx *c) {
+// Stage A; with dt, the dt reduction in it.
+int run_stage_a(wx_ctx *c, bool dt = false) {
   ProfScope ps(c, KID_STAGEA);
-  int rc = launch_stageA(c->dP.ptr, c->neq, c->queue(), c->nleaf(), 512, 0, c->cur_u(), c->other_u(), c->pc(),
+  QueueRef q = c->queue();
+  if (dt) q.stat = c->dStat.ptr;
+  int rc = launch_stageA(c->dP.ptr, c->neq, q, c->nleaf(), 512, 0, c->cur_u(), c->other_u(), c->pc(),
                          c->dS.ptr, c->stream);
   if (rc) return fail(rc, "stage launch failed: %s", hipGetErrorString(hipGetLastError()));
   return WX_OK;
@@ -820,13 +828,15 @@ int wx_step(wx_ctx *c, int32_t nsteps, int32_t do_admesh_flag, double *time, dou
     int rc = split ? tables_leaves(c) : WX_OK;
     if (!rc) rc = update_stats(c);
     if (rc) return rc;
+    const bool few = c->nleaf() >= 1 && c->nleaf() <= kFewLeaves;
     {
       ProfScope ps(c, KID_DTRED);      // timestep; time += dt
-      rc = launch_dtreduce(c->dP.ptr, c->tLeaves, c->dStat.ptr, c->tOff, 1, c->dS.ptr, 1, c->stream);
+      rc = launch_dtreduce(c->dP.ptr, c->tLeaves, c->dStat.ptr, c->tOff, 1, c->dS.ptr, few ? kDtInStageA : 1,
+                           c->stream);
     }
     if (rc) return fail(rc, "dtreduce launch failed");
     z += (double)c->nleaf() * NX * NY;
-    rc = run_stage_a(c);               // tstep
+    rc = run_stage_a(c, few);          // tstep
     if (!rc && split) rc = tables_ops(c);
     if (!rc) rc = run_stages_bf(c);
     if (rc) return rc;

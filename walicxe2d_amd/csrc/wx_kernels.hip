@@ -357,7 +357,10 @@ __device__ __forceinline__ void cyl_source(const wx_params *__restrict__ p, cons
 // Stage A: src/tstep.f90:22-46 (hllcfluxes choice 1 + step with dt/2).
 // MILD: the short divisions where they hold (wx_physics.h), and the cells'
 // sound speeds taken once per cell instead of once per face and side.
-template <int NEQ, int BS, bool PERSIST, bool MILD>
+// DT: the step's dt too (k_dtreduce with advance), at most BS blocks of one
+// instance: every workgroup takes it from all blocks' partials, in the order
+// k_dtreduce takes, and workgroup 0 writes it.
+template <int NEQ, int BS, bool PERSIST, bool MILD, bool DT = false>
 __device__ __forceinline__ void stageA_body(const wx_params *__restrict__ P, QueueRef q, const double *__restrict__ U,
                                             double *__restrict__ Q, const double *__restrict__ Pc,
                                             DevScalars *__restrict__ Sa) {
@@ -366,6 +369,7 @@ __device__ __forceinline__ void stageA_body(const wx_params *__restrict__ P, Que
   __shared__ double G[NEQ * 272];
   __shared__ double cst[MILD ? 18 * NP : 1];   // sound speeds of rows 0..17
   __shared__ uint32_t votes[BS / 64];
+  __shared__ double dtw[2][BS / 64];   // DT: the waves' minima
   const int wave = wave_of();
   // the first entry's record is read together with the queue length
   const int b0 = PERSIST ? (int)blockIdx.x : xcd_entry(blockIdx.x, gridDim.x);
@@ -384,6 +388,20 @@ __device__ __forceinline__ void stageA_body(const wx_params *__restrict__ P, Que
   // cooling left (the reference's primit, src/coolingdmc.f90:27-38 and
   // src/tstep.f90:27-36), not the one u gives back.
   const bool carried = Pc && p->cooling == 2;
+  if constexpr (DT) {
+    const int tid = tid_again(wave);
+    double a = 1.e30, c = 1e30;
+    if (tid < nleaf) {
+      const int id = q.rec[tid].id;
+      a = dmin(a, q.stat[2 * id]);
+      c = dmin(c, q.stat[2 * id + 1]);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      a = dmin(a, __shfl_xor(a, o));
+      c = dmin(c, __shfl_xor(c, o));
+    }
+    if ((tid & 63) == 0) { dtw[0][wave] = a; dtw[1][wave] = c; }
+  }
   const double *pcb = carried ? Pc + (size_t)L.id * NC : nullptr;
   const bool pok = MILD && mild_params(p, L.level);
   bool ok = pok;
@@ -435,8 +453,31 @@ __device__ __forceinline__ void stageA_body(const wx_params *__restrict__ P, Que
   else err = flux_sweep<NEQ, 1, BS>(p, wave, prim, F, G, nullptr);
   __syncthreads();
   const int tid = tid_again(wave);
+  double dt;
+  if constexpr (DT) {
+    double a = dtw[0][0], c = dtw[1][0];
+#pragma unroll
+    for (int k = 1; k < BS / 64; ++k) { a = dmin(a, dtw[0][k]); c = dmin(c, dtw[1][k]); }
+    if (BS < 1024) { a = dmin(a, 1.e30); c = dmin(c, 1e30); }   // k_dtreduce's waves without a block
+    dt = dmin(p->cfl * a, 0.4 * c * p->Psc / p->tsc);
+    // written by a thread past the cells'
+    if (blockIdx.x == 0 && tid == BS - 1) {
+      S->dtp_min = a;
+      S->dtcool_min = c;
+      S->dt = dt;
+      const double t = S->time + dt;
+      S->time = t;
+      if (p->otherb) {
+        S->vjet = jet_velocity(p, t);
+        S->vjet_time = t;
+        S->vjet_ok = 1;
+      }
+    }
+  } else {
+    dt = S->dt;
+  }
   if (tid < 256) {   // one thread per interior cell
-    const double dtm = S->dt / 2.;
+    const double dtm = dt / 2.;
     double dtdx, dtdy;
     dt_over_dx(p, pok, dtm, L.level, dtdx, dtdy);
     const int i = tid % 16 + 1, j = tid / 16 + 1;
@@ -469,6 +510,13 @@ __global__ __launch_bounds__(BS, PERSIST ? 1 : 8) void k_stageA(const wx_params 
                                                 const double *__restrict__ U, double *__restrict__ Q,
                                                 const double *__restrict__ Pc, DevScalars *__restrict__ Sa) {
   stageA_body<NEQ, BS, PERSIST, false>(P, q, U, Q, Pc, Sa);
+}
+// For the few blocks it serves (wx_host.cpp) two workgroups a compute unit are enough.
+template <int NEQ>
+__global__ __launch_bounds__(512, 4) void k_stageA_dt(const wx_params *__restrict__ P, QueueRef q,
+                                                const double *__restrict__ U, double *__restrict__ Q,
+                                                const double *__restrict__ Pc, DevScalars *__restrict__ Sa) {
+  stageA_body<NEQ, 512, false, false, true>(P, q, U, Q, Pc, Sa);
 }
 template <int NEQ, int BS>
 __global__ __launch_bounds__(BS, 8) void k_stageA_mild(const wx_params *__restrict__ P, QueueRef q,
@@ -1398,6 +1446,11 @@ constexpr int kMildA = 1024, kMildB = 3000;
 int launch_stageA(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const double *U,
                   double *Q, const double *Pc, DevScalars *S, hipStream_t stream) {
   if (grid <= 0) return WX_OK;
+  if (q.stat) {   // with the dt reduction
+    if (persist || bs != 512 || grid > 512) return WX_EARG;
+    WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageA_dt<N>), dim3(grid), dim3(512), 0, stream, P, q, U, Q, Pc, S));
+    return hip_status();
+  }
   if (!persist && grid >= kMildA) {
     WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageA_mild<N, B>), dim3(grid), dim3(B), 0, stream, P, q, U, Q, Pc, S)));
     return hip_status();
@@ -1463,7 +1516,7 @@ int launch_blockstat(const wx_params *P, int neq, const LeafRec *leaves, int nle
 
 int launch_dtreduce(const wx_params *P, const LeafRec *rec, const double *stat, const int32_t *inst_off,
                     int ninst, DevScalars *S, int advance, hipStream_t stream) {
-  if (ninst <= 0) return WX_OK;
+  if (ninst <= 0 || advance == kDtInStageA) return WX_OK;
   hipLaunchKernelGGL(k_dtreduce, dim3(ninst), dim3(1024), 0, stream, P, rec, stat, inst_off, S, advance);
   return hip_status();
 }
