@@ -386,7 +386,7 @@ int sync_scalars(wx_ctx *c) {
 // Up to there stage A also takes the dt reduction, a launch of one workgroup
 // that costs 4-5 us by itself against about 2 us in stage A (a trip for the
 // leaf records and one for their partials): explosion, 16 blocks, 22.2 / 18.7
-// us per step, jet of about 450 with the hybrid solver 63.9 / 62.3; above, a
+// us per step, jet of 37x11 roots with the hybrid solver 63.9 / 62.3; above, a
 // thread would take several records.
 constexpr int kFewLeaves = 512;
 

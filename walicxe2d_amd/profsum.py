@@ -13,8 +13,8 @@ that `rocprofv3 -d DIR -o NAME` writes).
         `--pmc FETCH_SIZE` / `--pmc WRITE_SIZE` runs, each counter scaled by
         what it reads for a plain device copy of --copy-mib MiB per dispatch.
 
-A hot-path kernel launches one workgroup per leaf block (of 256 threads, or
-512 for stage A), so its workgroup count times the 256 interior cells of a
+A hot-path kernel launches one workgroup per leaf block (of 128 to 512
+threads), so its workgroup count times the 256 interior cells of a
 block is the zone-updates of that launch.
 """
 from __future__ import annotations
@@ -120,6 +120,7 @@ def _per_kernel(db: str):
 
 def traffic(copy_fetch: str, copy_write: str, fetch: str, write: str, copy_mib: int) -> dict:
     out = {"factors": {}, "bytes_per_zone_update": {}}
+    sums = {}
     for ctr, cdb, kdb in (("FETCH_SIZE", copy_fetch, fetch), ("WRITE_SIZE", copy_write, write)):
         cp = _per_kernel(cdb)
         kib = [v[0] / v[1] for k, v in cp.items() if "copyBuffer" in k or "elementwise" in k.lower()]
@@ -128,9 +129,13 @@ def traffic(copy_fetch: str, copy_write: str, fetch: str, write: str, copy_mib: 
         fac = copy_mib * 1024 / max(kib)
         out["factors"][ctr] = fac
         for k, (tot, n, gs) in _per_kernel(kdb).items():
-            s = short(k).split("<")[0]
+            s = short(k).split("<")[0].removesuffix("_mild")   # both forms of a stage count as one kernel
             if s in HOT:
-                out["bytes_per_zone_update"].setdefault(s, {})[ctr] = tot * 1024 * fac / gs
+                a = sums.setdefault((s, ctr), [0.0, 0])
+                a[0] += tot * 1024 * fac
+                a[1] += gs
+    for (s, ctr), (tot, gs) in sums.items():
+        out["bytes_per_zone_update"].setdefault(s, {})[ctr] = tot / gs
     return out
 
 
