@@ -1,0 +1,77 @@
+// Sequences of calls a host program makes, through the product's host runtime
+// built against the host-only HIP stand-in.  TEST SCAFFOLDING.
+//   host_calls_check CHECK
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "../../include/wx_capi.h"
+#include "../../walicxe2d_amd/csrc/wx_runtime.h"
+#include "fake_kernels.cpp"
+
+#define REQUIRE(x)                                              \
+  do {                                                          \
+    if (!(x)) {                                                 \
+      char b[512] = "";                                         \
+      wx_last_error(b, 512);                                    \
+      fprintf(stderr, "line %d: %s (%s)\n", __LINE__, #x, b);   \
+      exit(1);                                                  \
+    }                                                           \
+  } while (0)
+
+static wx_params params(int rx, int ry, int nlevs, int nblocks, int otherb) {
+  wx_params p{};
+  p.neq = 4; p.nlevs = nlevs; p.nbrootx = rx; p.nbrooty = ry; p.nblocks = nblocks; p.otherb = otherb;
+  p.cv = 1.5; p.gamma = 5. / 3.; p.cfl = 0.4; p.tol = 0.05; p.tol2 = 1.0;
+  p.Tempsc = 1; p.Psc = 1; p.tsc = 1;
+  for (int l = 0; l < nlevs; ++l) p.dx[l] = p.dy[l] = 1.0 / (16 * rx) / (1 << l);
+  return p;
+}
+
+static wx_ctx *context(const wx_params &p) {
+  wx_ctx *c = nullptr;
+  REQUIRE(wx_create(&p, &c) == WX_OK);
+  std::vector<double> u((size_t)(p.nbrootx * p.nbrooty + 1) * p.neq * 400, 1.0);
+  REQUIRE(wx_basegrid(c, u.data(), p.nbrootx * p.nbrooty) == WX_OK);
+  return c;
+}
+
+struct Tables {
+  std::vector<int32_t> rec, o2, o1;
+  bool operator==(const Tables &t) const { return rec == t.rec && o2 == t.o2 && o1 == t.o1; }
+};
+static Tables tables(wx_ctx *c) {
+  int32_t n = 0;
+  REQUIRE(wx_get_tables(c, &n, nullptr, nullptr, nullptr, 0) == WX_OK);
+  Tables t{std::vector<int32_t>((size_t)n * 8), std::vector<int32_t>((size_t)n * 16), std::vector<int32_t>((size_t)n * 16)};
+  REQUIRE(wx_get_tables(c, &n, t.rec.data(), t.o2.data(), t.o1.data(), n) == WX_OK);
+  return t;
+}
+
+// A list from the host that leaves segments uncovered is refused; the
+// library's own list afterwards gives the tables it gave before, the jet
+// imposition flags of the leaf records included.
+static void rejected_list() {
+  for (int builder : {0, 1}) {
+    wx_ctx *c = context(params(4, 3, 2, 100, 1));
+    REQUIRE(wx_set_builder(c, builder) == WX_OK);
+    REQUIRE(wx_locatebounds(c, nullptr) == WX_OK);
+    const Tables want = tables(c);
+    int flagged = 0;
+    for (size_t l = 0; l < want.rec.size() / 8; ++l) flagged += want.rec[l * 8 + 4] & 1;
+    REQUIRE(flagged > 0);
+    REQUIRE(wx_set_bounds(c, nullptr, 0, 0) != WX_OK);
+    REQUIRE(wx_locatebounds(c, nullptr) == WX_OK);
+    REQUIRE(tables(c) == want);
+    wx_destroy(c);
+  }
+}
+
+int main(int argc, char **argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "rejected_list") rejected_list();
+  else return 2;
+  return 0;
+}

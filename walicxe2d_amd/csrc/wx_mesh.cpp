@@ -171,6 +171,10 @@ int compile_ops(Mesh *c) {
   const size_t nseg = (size_t)nleaf * 8;
   const bool otherb = c->p.otherb != 0;
   const bool outfyb_bug = lb_outfyb(c->p) != 0;
+  // current again at the end: a list that is refused on the way may have set
+  // some records' imposition flags, and an external list's are not the tree's
+  const bool records = c->leaves_ok && !c->bounds_external;
+  c->leaves_ok = c->ops_ok = false;
   // Fills I and II receive the same writes except for the OUTFYB entries of
   // boundaryI (src/boundaryI.f90:87: a bottom box entry writes block e + 1
   // instead of its own block): fill II is compiled from the list without
@@ -285,9 +289,8 @@ int compile_ops(Mesh *c) {
     if ((o2[k].y & 15) == GK_NONE)
       return fail(WX_EARG, "boundaryII: block %d ghost segment %d not covered by the list",
                   c->leaves[k / 8].id, (int)(k % 8));
-  if (c->bounds_external) {
-    c->leaves_ok = false;   // their imposition flags are that list's
-  } else {
+  c->leaves_ok = records;
+  if (!c->bounds_external) {
     if (c->idOps.size() < ((size_t)c->cap + 1) * 8) c->idOps.resize(((size_t)c->cap + 1) * 8);
     for (int l = 0; l < nleaf; ++l) memcpy(&c->idOps[(size_t)c->leaves[l].id * 8], o2 + (size_t)l * 8, 8 * sizeof(int2));
     c->ops_ok = true;
