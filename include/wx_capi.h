@@ -115,8 +115,8 @@ int wx_locatebounds(wx_ctx *ctx, int32_t *ninternal);
  * and stage A; 0 on the host (the list itself, compiled, then uploaded);
  * 2 on the device with the scan over block IDs spread over many workgroups
  * at any mesh size (the form it takes above 2048 IDs); 3 (default) by size:
- * on the device from 16384 leaves up, or from 3072 after a change that
- * rewrote much of the tree, else on the host.  All give identical
+ * on the device from 16384 leaves up, or from 6144 after a change that
+ * rewrote much of the tree (or all: one from the host), else on the host.  All give identical
  * tables.  A list set by wx_set_bounds is always compiled on the host. */
 int wx_set_builder(wx_ctx *ctx, int32_t on_device);
 /* The current gather tables, for checks: *nleaf leaf records (8 int32 each:

@@ -9,7 +9,20 @@
 
 #include "../../include/wx_capi.h"
 #include "../../walicxe2d_amd/csrc/wx_runtime.h"
+#include "../../walicxe2d_amd/csrc/wx_surrogate.h"
+
+#define launch_build_tables launch_build_tables_cpu
 #include "fake_kernels.cpp"
+#undef launch_build_tables
+
+static int g_builds = 0;   // launches of the device table builder
+namespace wx {
+int launch_build_tables(const wx_params &p, const TreeRow *T, int nbmax, int nleaf_host, LbInfo *info, LbPart *part,
+                        LbOut out, int wide, DevScalars *S, hipStream_t st) {
+  ++g_builds;
+  return launch_build_tables_cpu(p, T, nbmax, nleaf_host, info, part, out, wide, S, st);
+}
+}  // namespace wx
 
 #define REQUIRE(x)                                              \
   do {                                                          \
@@ -17,7 +30,7 @@
       char b[512] = "";                                         \
       wx_last_error(b, 512);                                    \
       fprintf(stderr, "line %d: %s (%s)\n", __LINE__, #x, b);   \
-      exit(1);                                                  \
+      _Exit(1);                                                 \
     }                                                           \
   } while (0)
 
@@ -69,9 +82,53 @@ static void rejected_list() {
   }
 }
 
+struct Tree {
+  int32_t nbmax = 0, nbleafs = 0;
+  std::vector<int32_t> lp, leaf, ic;
+};
+static Tree tree(wx_ctx *c) {
+  Tree t;
+  REQUIRE(wx_info(c, &t.nbmax, &t.nbleafs, nullptr) == WX_OK);
+  t.lp.resize((size_t)t.nbmax * 8);
+  t.leaf.resize(t.nbmax);
+  t.ic.resize((size_t)t.nbmax * 2);
+  REQUIRE(wx_get_tree(c, t.lp.data(), t.leaf.data(), t.ic.data(), t.nbmax, &t.nbmax, &t.nbleafs) == WX_OK);
+  return t;
+}
+static int upload_tree(wx_ctx *c, const Tree &t) {
+  return wx_upload_tree(c, t.lp.data(), t.leaf.data(), t.ic.data(), t.nbmax, t.nbmax, t.nbleafs);
+}
+
+// Where the ops are built by default: a tree that is new as a whole counts as
+// a change that rewrote much of it (on the device from 6 144 leaves up), a
+// change of a few rows does not.
+static void builder_of_new_trees() {
+  for (int ry : {95, 96}) {   // 6 080 and 6 144 roots
+    const int dev = ry == 96;
+    wx_ctx *c = context(params(64, ry, 2, 64 * ry + 400, 0));
+    g_builds = 0;
+    REQUIRE(wx_locatebounds(c, nullptr) == WX_OK);
+    REQUIRE(g_builds == dev);
+    Tree t = tree(c);
+    for (int32_t &x : t.ic) x += 16;
+    REQUIRE(upload_tree(c, t) == WX_OK);
+    REQUIRE(wx_locatebounds(c, nullptr) == WX_OK);
+    REQUIRE(g_builds == 2 * dev);
+    std::vector<signed char> f(64 * ry + 1, 0);
+    f[70] = 1;
+    wxsim_set_flags(f.data(), (int)f.size());
+    int32_t changed = 0;
+    REQUIRE(wx_admesh(c, &changed) == WX_OK && changed == 1);
+    REQUIRE(wx_locatebounds(c, nullptr) == WX_OK);
+    REQUIRE(g_builds == 2 * dev);
+    wx_destroy(c);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "rejected_list") rejected_list();
+  else if (what == "builder_of_new_trees") builder_of_new_trees();
   else return 2;
   return 0;
 }

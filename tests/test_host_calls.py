@@ -38,3 +38,7 @@ def _run(exe, check):
 
 def test_own_list_after_a_rejected_one(program):
     _run(program, "rejected_list")
+
+
+def test_builder_of_new_trees(program):
+    _run(program, "builder_of_new_trees")

@@ -107,10 +107,13 @@ int arena_fit(wx_ctx *c) {
 // device runs the dt reduction and stage A, and that is the faster of the two
 // up to some 16 000 leaves (us/step, host / device: supernova, 544 leaves
 // 61 / 77; jets, 1 177 92 / 108; 5 319 197 / 205; 9 261 309 / 312; 16 426
-// 573 / 575; 25 633 882 / 875).  A change that rewrites a large part of the
-// tree has the host compile all of it, about 60 ns a leaf, of which stage A
-// hides 8: there the device takes over at 3 072.
-constexpr size_t kDeviceBuilderLeaves = 16384, kDeviceBuilderMany = 3072;
+// 573 / 575; 25 633 882 / 875).  After a change that rewrites a large part of
+// the tree, or a new tree from the host, the host compiles all of it: there the
+// device takes over earlier (us for a new tree, wx_locatebounds and
+// wx_timestep, or a step of wx_step, host / device: 1 998 leaves 101 / 155,
+// 164 / 179; 3 078 134 / 179, 217 / 235; 5 262 210 / 227, 318 / 329; 6 478
+// 247 / 264, 372 / 375; 7 758 291 / 273, 432 / 427; 10 318 367 / 329, 552 / 541).
+constexpr size_t kDeviceBuilderLeaves = 16384, kDeviceBuilderMany = 6144;
 
 bool use_device_builder(const wx_ctx *c) {
   if (c->dev_builder == 0 || c->bounds_external) return false;

@@ -352,10 +352,10 @@ static bool next_to(Mesh *c, int n) {
 }
 
 int update_leaves(Mesh *c) {
-  // many rows at once: the full passes read memory in order (a jet of 1 024
+  // many rows at once, or a new tree: the full passes read memory in order (a jet of 1 024
   // blocks, us from the rows / full: 0.10 written rows a leaf 34 / 70, 0.17
   // 55 / 71, 0.27 81 / 80, 0.42 121 / 89)
-  c->many_rows = c->leaves_ok && c->newRows.size() > c->leaves.size() / 4;
+  c->many_rows = !c->leaves_ok || c->newRows.size() > c->leaves.size() / 4;
   if (!c->leaves_ok || c->bounds_external || c->many_rows) return compile_leaves(c);
   const int nbmax = c->nbmax;
   const bool otherb = c->p.otherb != 0, counts = otherb || lb_outfyb(c->p), ops = c->ops_ok;

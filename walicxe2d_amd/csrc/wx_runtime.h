@@ -111,7 +111,7 @@ struct Mesh {
   std::vector<int2> idOps;
   std::vector<uint8_t> idCnt;  // list entries of every leaf, where its flag or the OUTFYB mode needs them
   bool leaves_ok = false, ops_ok = false, ops_pending_id = false, reops_all = true, binfo_all = true;
-  bool many_rows = false;   // the last change wrote too many rows for that
+  bool many_rows = false;   // the last change wrote too many rows for that, or the whole tree
   // fill II's ops of leaf l, wherever they are current
   const int2 *leaf_ops(size_t l) const { return ops_ok ? &idOps[(size_t)leaves[l].id * 8] : &opsII[l * 8]; }
 
