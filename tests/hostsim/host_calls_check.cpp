@@ -125,10 +125,29 @@ static void builder_of_new_trees() {
   }
 }
 
+// wx_info's list length after an upload of a tree that nothing has looked at
+// yet: no pointer of it is followed.
+static void info_of_an_unchecked_tree() {
+  wx_ctx *c = context(params(6, 5, 2, 200, 0));
+  REQUIRE(wx_locatebounds(c, nullptr) == WX_OK);
+  std::vector<signed char> f(201, 0);
+  f[8] = 1;
+  wxsim_set_flags(f.data(), (int)f.size());
+  int32_t changed = 0, nbmax = 0, nbleafs = 0, n = 0;
+  REQUIRE(wx_admesh(c, &changed) == WX_OK && changed == 1);
+  REQUIRE(wx_locatebounds(c, nullptr) == WX_OK);   // brought up to date without the list
+  Tree t = tree(c);
+  for (int k = 4; k < 8; ++k) t.lp[(size_t)k * t.nbmax + 2] = 1 << 28;
+  REQUIRE(upload_tree(c, t) == WX_OK);
+  REQUIRE(wx_info(c, &nbmax, &nbleafs, &n) == WX_OK && nbmax == 34 && nbleafs == 33);
+  wx_destroy(c);
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "rejected_list") rejected_list();
   else if (what == "builder_of_new_trees") builder_of_new_trees();
+  else if (what == "info_of_an_unchecked_tree") info_of_an_unchecked_tree();
   else return 2;
   return 0;
 }

@@ -42,3 +42,7 @@ def test_own_list_after_a_rejected_one(program):
 
 def test_builder_of_new_trees(program):
     _run(program, "builder_of_new_trees")
+
+
+def test_info_of_an_unchecked_tree(program):
+    _run(program, "info_of_an_unchecked_tree")

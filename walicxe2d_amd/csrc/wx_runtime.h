@@ -134,6 +134,7 @@ struct Mesh {
     dirtyRows.clear();
     allDirty = true;
     leaves_ok = ops_ok = ops_pending_id = false;
+    list_stale = false;   // located again with the new tree's tables, not from rows nothing has looked at
   }
   void init(const wx_params &pp);
 };
