@@ -86,7 +86,8 @@ int wx_destroy(wx_ctx *ctx);
  * (src/globals.f90:13-18, column-major, ld = leading dimension = number of
  * rows of lp/icoord/leaf arrays, rows indexed by block ID - 1).
  * Replaces nothing in the reference (its arrays are already in memory);
- * this is the transpose into the device's [id][var][j][i] tiles. */
+ * this is the transpose into the device's tiles, [id][var][cell], the cells
+ * in an order of their own (interior, ghost layers 1 and 2, corners). */
 int wx_upload(wx_ctx *ctx, const double *u, int32_t layout, const int32_t *lp,
               const int32_t *leaf, const int32_t *icoord, int32_t ld,
               int32_t nbmax, int32_t nbleafs);

@@ -152,7 +152,21 @@ int launch_meshops(const wx_params *P, int, const MeshOp *ops, int nops, double 
   });
   return 0;
 }
-int launch_transpose(int, int, const double *, double *, int, int, hipStream_t) { return 0; }
+int launch_transpose(int neq, int cap, const double *src, double *dst, int mode, int, hipStream_t st) {
+  if (mode < 2) return 0;
+  hipsim::launch(st, {src, dst}, [=] {   // as k_reorder
+    for (size_t v = 0; v < (size_t)cap * neq; ++v) {
+      double t[NC];
+      memcpy(t, src + v * NC, sizeof t);
+      for (int c = 0; c < NC; ++c) {
+        const int d = tile_cell(c % NP - 1, c / NP - 1);
+        if (mode == 3) dst[v * NC + c] = t[d];
+        else dst[v * NC + d] = t[c];
+      }
+    }
+  });
+  return 0;
+}
 int launch_h2d(const CopyDesc *d, int n, hipStream_t st) {
   hipsim::launch(st, {d}, [=] {
     for (int k = 0; k < n; ++k) memmove(d[k].dst, d[k].src, d[k].bytes);

@@ -5,6 +5,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/wx_capi.h"
@@ -12,11 +13,22 @@
 #include "../../walicxe2d_amd/csrc/wx_surrogate.h"
 
 #define launch_build_tables launch_build_tables_cpu
+#define launch_transpose launch_transpose_cpu
 #include "fake_kernels.cpp"
 #undef launch_build_tables
+#undef launch_transpose
 
 static int g_builds = 0;   // launches of the device table builder
+static const double *g_state = nullptr;   // tiles that no launch may write, and how many values
+static size_t g_nstate = 0;
 namespace wx {
+int launch_transpose(int neq, int cap, const double *src, double *dst, int mode, int ld, hipStream_t st) {
+  if (g_state && dst >= g_state && dst < g_state + g_nstate) {
+    fprintf(stderr, "a launch writes the state\n");
+    _Exit(1);
+  }
+  return launch_transpose_cpu(neq, cap, src, dst, mode, ld, st);
+}
 int launch_build_tables(const wx_params &p, const TreeRow *T, int nbmax, int nleaf_host, LbInfo *info, LbPart *part,
                         LbOut out, int wide, DevScalars *S, hipStream_t st) {
   ++g_builds;
@@ -143,11 +155,45 @@ static void info_of_an_unchecked_tree() {
   wx_destroy(c);
 }
 
+// A download, of any size, reads the state and nothing else of it: no launch
+// writes the tiles, and two threads may download one context at once.
+static void downloads() {
+  for (int n : {1, 4, 80, 81, 82, 2700}) {   // states below and above 1 MiB (12.8 KB a block), and above 32 MiB
+    wx_params p = params(n, 1, 1, n, 0);
+    wx_ctx *c = context(p);
+    Tree t = tree(c);
+    const size_t m = (size_t)(n + 1) * p.neq * 400;
+    std::vector<double> u(m), got[2];
+    for (size_t k = 0; k < m; ++k) u[k] = (double)(k * 2654435761u % 1000003u);
+    REQUIRE(wx_upload(c, u.data(), WX_LAYOUT_BLOCK, t.lp.data(), t.leaf.data(), t.ic.data(), n, n, n) == WX_OK);
+    // the tiles: the one allocation that holds exactly the uploaded interior cell
+    for (const auto &a : hipsim::allocs)
+      if (a.second == m * sizeof(double) && ((const double *)a.first)[p.neq * 400] == u[p.neq * 400 + 2 * 20 + 2]) {
+        g_state = (const double *)a.first;
+        g_nstate = m;
+      }
+    REQUIRE(g_state);
+    for (int rep = 0; rep < 2; ++rep) {
+      std::thread th[2];
+      for (int k = 0; k < 2; ++k)
+        th[k] = std::thread([&, k] {
+          got[k].assign(m, 0.0);
+          for (int r = 0; r < (n < 100 ? 40 : 2); ++r)
+            REQUIRE(wx_download(c, got[k].data(), nullptr, WX_LAYOUT_BLOCK, 0) == WX_OK && got[k] == u);
+        });
+      for (std::thread &x : th) x.join();
+    }
+    g_state = nullptr;
+    wx_destroy(c);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "rejected_list") rejected_list();
   else if (what == "builder_of_new_trees") builder_of_new_trees();
   else if (what == "info_of_an_unchecked_tree") info_of_an_unchecked_tree();
+  else if (what == "downloads") downloads();
   else return 2;
   return 0;
 }

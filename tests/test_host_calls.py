@@ -31,6 +31,11 @@ def program(tmp_path_factory):
     return _build(tmp_path_factory, "address,undefined")
 
 
+@pytest.fixture(scope="module")
+def program_tsan(tmp_path_factory):
+    return _build(tmp_path_factory, "thread")
+
+
 def _run(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr[-4000:]
@@ -46,3 +51,8 @@ def test_builder_of_new_trees(program):
 
 def test_info_of_an_unchecked_tree(program):
     _run(program, "info_of_an_unchecked_tree")
+
+
+def test_downloads_only_read(program, program_tsan):
+    _run(program, "downloads")
+    _run(program_tsan, "downloads")

@@ -574,13 +574,7 @@ int grp_basegrid(EnsGroup *e, int32_t inst, const double *uroots, int32_t nroots
   m.pc_stale = true;
   e->binfo_dev[inst] = 0;
   e->shadow[inst].valid = false;
-  const size_t bytes = (size_t)(nroots + 1) * e->tile() * sizeof(double);
-  double *u = e->cur_u() + (size_t)e->slotbase[inst] * e->tile();
-  HIPCHK(hipMemcpyAsync(u, uroots, bytes, hipMemcpyHostToDevice, e->stream));
-  rc = launch_transpose(e->neq, nroots + 1, u, u, 2, 0, e->stream);
-  if (rc) return fail(rc, "reorder launch failed");
-  HIPCHK(hipStreamSynchronize(e->stream));
-  return WX_OK;
+  return tiles_to_device(e, uroots, (size_t)nroots + 1, e->neq, e->cur_u() + (size_t)e->slotbase[inst] * e->tile());
 }
 
 int grp_admesh(EnsGroup *e, int32_t *changed) {

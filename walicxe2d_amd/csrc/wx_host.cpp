@@ -598,10 +598,7 @@ int wx_upload(wx_ctx *c, const double *u, int32_t layout, const int32_t *lp, con
   c->stats_all_stale = true;
   c->pc_stale = true;
   if (layout == WX_LAYOUT_BLOCK) {
-    const size_t n = (size_t)(nbmax + 1) * c->neq * NC;
-    HIPCHK(hipMemcpyAsync(c->cur_u(), u, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    rc = launch_transpose(c->neq, nbmax + 1, c->cur_u(), c->cur_u(), 2, 0, c->stream);
-    if (rc) return fail(rc, "reorder launch failed");
+    return tiles_to_device(c, u, (size_t)nbmax + 1, c->neq, c->cur_u());
   } else if (layout == WX_LAYOUT_FORTRAN) {
     if (ld > c->cap) return fail(WX_EARG, "ld %d exceeds capacity %d", ld, c->cap);
     const size_t n = (size_t)ld * c->neq * NC;
@@ -632,11 +629,10 @@ int wx_download(wx_ctx *c, double *u, double *prim, int32_t layout, int32_t ld_i
   if (!c) return fail(WX_EARG, "null context");
   int rc;
   HIPCHK(hipStreamSynchronize(c->stream));
-  const size_t n = (size_t)(c->nbmax + 1) * c->neq * NC;
   for (int pass = 0; pass < 2; ++pass) {
     double *dst = pass == 0 ? u : prim;
     if (!dst) continue;
-    double *src = c->cur_u();
+    const double *src = c->cur_u();
     if (pass == 1) {
       if ((rc = c->dScratch.ensure((size_t)(c->cap + 1) * c->neq * NC))) return rc;
       rc = launch_calcprim(c->dP.ptr, c->neq, c->nbmax, c->cur_u(), c->dScratch.ptr, c->stream);
@@ -794,12 +790,7 @@ int wx_basegrid(wx_ctx *c, const double *uroots, int32_t nroots) {
   int rc = basegrid_tree(c);
   if (rc) return rc;
   c->pc_stale = true;
-  const size_t n = (size_t)(nroots + 1) * c->neq * NC;
-  HIPCHK(hipMemcpyAsync(c->cur_u(), uroots, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  rc = launch_transpose(c->neq, nroots + 1, c->cur_u(), c->cur_u(), 2, 0, c->stream);
-  if (rc) return fail(rc, "reorder launch failed");
-  HIPCHK(hipStreamSynchronize(c->stream));
-  return WX_OK;
+  return tiles_to_device(c, uroots, (size_t)nroots + 1, c->neq, c->cur_u());
 }
 
 int wx_admesh(wx_ctx *c, int32_t *changed) {

@@ -1354,21 +1354,24 @@ __global__ void k_transpose(int cap, const double *__restrict__ src, double *__r
   }
 }
 
-// The cells of one tile variable per 128 threads reordered in place, between
-// padded host rows and the device's order.
-__global__ __launch_bounds__(256) void k_reorder(size_t ntile, double *__restrict__ u, int to_rows) {
+// The cells of one tile variable per 128 threads reordered, between padded
+// host rows and the device's order; src may be dst.  Either side can be mapped
+// host memory: both are read and written in the order of memory, the tile
+// turned over in LDS.
+__global__ __launch_bounds__(256) void k_reorder(size_t ntile, const double *src, double *dst, int to_rows) {
   __shared__ double t[2][NC];
   const int h = threadIdx.x >> 7, l = threadIdx.x & 127;
   const size_t v = (size_t)blockIdx.x * 2 + h;
-  double *b = u + v * NC;
   if (v < ntile)
-    for (int c = l; c < NC; c += 128) t[h][c] = b[c];
+    for (int c = l; c < NC; c += 128) {
+      const int d = to_rows ? c : tile_cell(c % NP - 1, c / NP - 1);
+      t[h][d] = src[v * NC + c];
+    }
   __syncthreads();
   if (v < ntile)
     for (int c = l; c < NC; c += 128) {
-      const int d = tile_cell(c % NP - 1, c / NP - 1);
-      if (to_rows) b[c] = t[h][d];
-      else b[d] = t[h][c];
+      const int d = to_rows ? tile_cell(c % NP - 1, c / NP - 1) : c;
+      dst[v * NC + c] = t[h][d];
     }
 }
 
@@ -1571,11 +1574,10 @@ int launch_h2d(const CopyDesc *d, int n, hipStream_t stream) {
 }
 
 int launch_transpose(int neq, int cap, const double *src, double *dst, int mode, int ld, hipStream_t stream) {
-  if (mode >= 2) {   // in place, cap tiles
-    if (src != dst) return WX_EARG;
+  if (mode >= 2) {   // cap tiles, one by one
     const size_t ntile = (size_t)cap * neq;
     if (ntile == 0) return WX_OK;
-    hipLaunchKernelGGL(k_reorder, dim3((unsigned)((ntile + 1) / 2)), dim3(256), 0, stream, ntile, dst, mode == 3);
+    hipLaunchKernelGGL(k_reorder, dim3((unsigned)((ntile + 1) / 2)), dim3(256), 0, stream, ntile, src, dst, mode == 3);
     return hip_status();
   }
   WX_DISPATCH(neq, hipLaunchKernelGGL(k_transpose<N>, dim3(1024), dim3(256), 0, stream, cap, src, dst, mode, ld));

@@ -199,6 +199,13 @@ struct Runtime {
   double prof_ms[NPROF] = {0};
   int64_t prof_n[NPROF] = {0};
 
+  // What state copies pass through (tiles_to_host, tiles_to_device): mapped
+  // pinned memory for small ones, device memory for a piece of a large
+  // download.  A download changes nothing but these, so it takes the lock.
+  char *xhost = nullptr, *xdev = nullptr;
+  DevBuf<double> xtiles;
+  std::mutex xmu;
+
   int create_stream();
   void destroy();
 };
@@ -219,10 +226,10 @@ const void *stage_inplace(Runtime *r, const void *src, size_t bytes);
 // Launches the round's copies and records the buffer's event.
 int stage_end(Runtime *r);
 void prof_collect(Runtime *r);
-// ntile device tiles from `tiles` on to host memory as padded rows: reordered
-// in place, copied and ordered back, so that no second buffer is needed.
-// Returns when the copy is done.
-int tiles_to_host(Runtime *r, double *tiles, size_t ntile, int neq, double *host);
+// ntile device tiles from `tiles` on to host memory as padded rows, and back;
+// the tiles are only read by the first.  Both return when the copy is done.
+int tiles_to_host(Runtime *r, const double *tiles, size_t ntile, int neq, double *host);
+int tiles_to_device(Runtime *r, const double *host, size_t ntile, int neq, double *tiles);
 
 int prof_report(Runtime *r, int32_t enable, double *ms, int64_t *counts, int32_t n);
 
