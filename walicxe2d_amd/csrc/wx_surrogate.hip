@@ -60,10 +60,10 @@ __global__ __launch_bounds__(256) void k_sur_feat(const SurDev *__restrict__ M, 
 }
 
 // Standardised inputs x[n][4] -> standardised outputs y[n][2]; a wave takes
-// 4 groups of 16 samples at a time.
+// G groups of 16 samples at a time.
+template <int G>
 __global__ __launch_bounds__(256) void k_sur_infer(const SurDev *__restrict__ M, const float *__restrict__ x,
                                                    int64_t n, float *__restrict__ y) {
-  constexpr int G = 4;
   const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
   const int64_t nset = (n + 16 * G - 1) / (16 * G);
   for (int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); b < nset; b += (int64_t)gridDim.x * 4) {
@@ -412,9 +412,18 @@ int launch_sur_feat(const SurDev *M, const double *in, int64_t n, float *f, floa
   return hip_ok();
 }
 
+// Up to one group of 16 samples for each of the card's 1 024 SIMDs, a wave takes
+// one: it lasts as long as its chain of four layers, which more groups lengthen.
+// Above, four share each weight operand's load.  us per wx_sur_infer_noalloc
+// with one / two / four groups a wave: 1 000 samples 11.5 / 12.5 / 14.4, 16 384
+// 11.6 / 12.6 / 14.6, 24 576 16.0 / 12.7 / 14.7, 65 536 24.8 / 17.0 / 14.6,
+// 262 144 77 / 44 / 35, 2 000 005 146 / 168 / 154.
+constexpr int64_t kInferOne = 16384;
+
 int launch_sur_infer(const SurDev *M, const float *x, int64_t n, float *y, hipStream_t stream) {
   if (n <= 0) return WX_OK;
-  hipLaunchKernelGGL(k_sur_infer, dim3(grid_for(n, 256)), dim3(256), 0, stream, M, x, n, y);
+  if (n <= kInferOne) hipLaunchKernelGGL(k_sur_infer<1>, dim3(grid_for(n, 64)), dim3(256), 0, stream, M, x, n, y);
+  else hipLaunchKernelGGL(k_sur_infer<4>, dim3(grid_for(n, 256)), dim3(256), 0, stream, M, x, n, y);
   return hip_ok();
 }
 
