@@ -1473,24 +1473,23 @@ int launch_stageB(const wx_params *P, int neq, QueueRef q, int grid, int bs, int
   return hip_status();
 }
 
-// Launches of tiles with n_HI from which the fill takes two waves per block
-// instead of four.  Its 320 cells are five passes of a wave: four waves take
+// Launches of tiles of five variables from which the fill takes two waves per
+// block instead of four.  Its 320 cells are five passes of a wave: four waves take
 // two rounds, three of them idle in the second (five of eight slots used), two
 // take three rounds (five of six), and ten such workgroups fill a compute unit
 // to the byte of LDS and at the same five waves per SIMD.  A block takes longer,
 // so it needs many rounds of blocks: passes of 5 322 blocks 80.3 -> 81.6 ms, of
 // ensembles without n_HI 125.5 -> 127.1, of two groups of 9 600 blocks
-// 297.4 -> 293.4.
+// 297.4 -> 293.4.  With six variables a tile is 19.6 KB, eight such workgroups
+// fit, and four waves per SIMD: 146 us against 143 on 10 930 blocks.
 constexpr int kFill128 = 8192;
 
 int launch_fillI_cool(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const int2 *ops,
                       const BlockRec *binfo, const double *Uin, double *Uout, double *stat, int8_t *flag,
                       DevScalars *S, FlagOut fo, double *Pc, hipStream_t stream) {
   if (grid <= 0) return WX_OK;
-  if (!persist && bs == 256 && neq >= 5 && grid >= kFill128) {
-    if (neq == 5) hipLaunchKernelGGL((k_fillI_cool<5, false, 128, false>), dim3(grid), dim3(128), 0, stream, P, q, ops, binfo, Uin, Uout, stat, flag, S, fo, nullptr, Pc);
-    else if (neq == 6) hipLaunchKernelGGL((k_fillI_cool<6, false, 128, false>), dim3(grid), dim3(128), 0, stream, P, q, ops, binfo, Uin, Uout, stat, flag, S, fo, nullptr, Pc);
-    else return WX_EARG;
+  if (!persist && bs == 256 && neq == 5 && grid >= kFill128) {
+    hipLaunchKernelGGL((k_fillI_cool<5, false, 128, false>), dim3(grid), dim3(128), 0, stream, P, q, ops, binfo, Uin, Uout, stat, flag, S, fo, nullptr, Pc);
     return hip_status();
   }
   WX_PERSIST_DISPATCH(persist, WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_fillI_cool<N, false, B, PS>), dim3(grid), dim3(B), 0, stream, P, q, ops, binfo, Uin, Uout, stat, flag, S, fo, nullptr, Pc))));
