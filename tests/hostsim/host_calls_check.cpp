@@ -14,14 +14,29 @@
 
 #define launch_build_tables launch_build_tables_cpu
 #define launch_transpose launch_transpose_cpu
+#define launch_stageA launch_stageA_cpu
+#define launch_stageB launch_stageB_cpu
 #include "fake_kernels.cpp"
 #undef launch_build_tables
 #undef launch_transpose
+#undef launch_stageA
+#undef launch_stageB
 
 static int g_builds = 0;   // launches of the device table builder
 static const double *g_state = nullptr;   // tiles that no launch may write, and how many values
 static size_t g_nstate = 0;
+static int g_stage[2] = {0, 0};   // stage launches, by whether the general form is asked for
 namespace wx {
+int launch_stageA(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const double *U, double *Uh,
+                  const double *Pc, DevScalars *S, hipStream_t st) {
+  ++g_stage[q.general != 0];
+  return launch_stageA_cpu(P, neq, q, grid, bs, persist, U, Uh, Pc, S, st);
+}
+int launch_stageB(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const int2 *ops,
+                  const BlockRec *binfo, double *U, double *Uh, DevScalars *S, hipStream_t st) {
+  ++g_stage[q.general != 0];
+  return launch_stageB_cpu(P, neq, q, grid, bs, persist, ops, binfo, U, Uh, S, st);
+}
 int launch_transpose(int neq, int cap, const double *src, double *dst, int mode, int ld, hipStream_t st) {
   if (g_state && dst >= g_state && dst < g_state + g_nstate) {
     fprintf(stderr, "a launch writes the state\n");
@@ -188,12 +203,41 @@ static void downloads() {
   }
 }
 
+// The stages are asked for their general form where a run's constants lie
+// outside the short divisions' range, on any level in use and in any instance.
+static void general_form() {
+  const double lo = 0x1p-64, hi = 0x1p64;
+  struct { double cv, Tempsc, dx1; int general; } k[] = {
+      {1.5, 1e4, 1.0, 0}, {lo, lo, lo, 0}, {1.5, hi, 1.0, 1}, {1.5, 1e4, hi, 1}, {0.99 * lo, 1e4, 1.0, 1}, {1.5, -1e4, 1.0, 1}};
+  for (const auto &x : k) {
+    wx_params p[2] = {params(2, 2, 2, 40, 0), params(2, 2, 2, 40, 0)};
+    p[1].cv = x.cv;
+    p[1].Tempsc = x.Tempsc;
+    p[1].dx[1] = x.dx1;
+    p[1].dx[2] = p[1].dy[3] = 1e300;   // levels not in use
+    g_stage[0] = g_stage[1] = 0;
+    wx_ctx *c = context(p[1]);
+    double t, dt, z;
+    REQUIRE(wx_step(c, 1, 0, &t, &dt, &z) == WX_OK);
+    REQUIRE(g_stage[x.general] == 2 && g_stage[!x.general] == 0);
+    wx_destroy(c);
+    wx_ens *e = nullptr;
+    REQUIRE(wx_ens_create(p, 2, &e) == WX_OK);
+    std::vector<double> u((size_t)5 * p[0].neq * 400, 1.0);
+    for (int i = 0; i < 2; ++i) REQUIRE(wx_ens_basegrid(e, i, u.data(), 4) == WX_OK);
+    REQUIRE(wx_ens_step(e, 1, 0, &z) == WX_OK);
+    REQUIRE(g_stage[x.general] == 4 && g_stage[!x.general] == 0);
+    wx_ens_destroy(e);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "rejected_list") rejected_list();
   else if (what == "builder_of_new_trees") builder_of_new_trees();
   else if (what == "info_of_an_unchecked_tree") info_of_an_unchecked_tree();
   else if (what == "downloads") downloads();
+  else if (what == "general_form") general_form();
   else return 2;
   return 0;
 }

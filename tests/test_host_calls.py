@@ -9,7 +9,7 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "..", "walicxe2d_amd", "csrc")
 SOURCES = [os.path.join(HERE, "hostsim", "host_calls_check.cpp")] + [
-    os.path.join(CSRC, f) for f in ("wx_host.cpp", "wx_mesh.cpp", "wx_runtime.cpp")]
+    os.path.join(CSRC, f) for f in ("wx_host.cpp", "wx_mesh.cpp", "wx_runtime.cpp", "wx_ensemble.cpp")]
 
 
 def _build(tmp_path_factory, sanitizers):
@@ -56,3 +56,7 @@ def test_info_of_an_unchecked_tree(program):
 def test_downloads_only_read(program, program_tsan):
     _run(program, "downloads")
     _run(program_tsan, "downloads")
+
+
+def test_general_form_of_the_stages(program):
+    _run(program, "general_form")

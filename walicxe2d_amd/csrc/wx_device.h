@@ -75,8 +75,18 @@ struct QueueRef {
   const QueueHdr *hdr;
   const LeafRec *rec;
   int32_t cap;
+  int32_t general;      // set where no block can take the stages' short divisions (short_forms)
   const double *stat;   // set where stage A takes the step's dt from the CFL partials itself
 };
+
+// The run's constants are in the range of the stages' short divisions
+// (mild_params of wx_physics.h, on every level).
+inline bool short_forms(const wx_params &p) {
+  auto in = [](double x) { return x >= 0x1p-64 && x < 0x1p64; };
+  bool ok = in(p.cv) && in(p.Tempsc) && in(p.gamma);
+  for (int l = 0; l < p.nlevs; ++l) ok = ok && in(p.dx[l]) && in(p.dy[l]);
+  return ok;
+}
 
 // launch_dtreduce's `advance` where the step's stage A takes dt: nothing to launch.
 constexpr int kDtInStageA = 2;

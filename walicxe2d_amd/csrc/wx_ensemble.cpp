@@ -61,6 +61,7 @@ struct EnsGroup : Runtime {
   // every instance, so they are neither uploaded nor gathered, and the fill
   // reads fill II's (fixed by the parameters for the ensemble's life)
   bool opsI_same_all = false;
+  bool general = false;   // an instance whose constants the stages' short divisions do not serve
   // block records on the device per instance: IDs 0 .. binfo_dev[i] - 1 (an
   // ID's level and position never change once created, so after a mesh
   // change only the IDs above the old maximum go up)
@@ -114,7 +115,7 @@ struct EnsGroup : Runtime {
   double *cur_u() { return U[cur].ptr; }
   double *other_u() { return U[cur ^ 1].ptr; }
   double *pc() { return dPc.ptr; }
-  QueueRef queue() const { return QueueRef{dQ.ptr, dRec.ptr, (int32_t)dRec.n}; }
+  QueueRef queue() const { return QueueRef{dQ.ptr, dRec.ptr, (int32_t)dRec.n, general, nullptr}; }
   size_t tile() const { return (size_t)neq * NC; }
 };
 
@@ -486,6 +487,7 @@ int grp_create(const wx_params *p, int32_t n, int nthreads, EnsGroup **out) {
   e->changed.resize(n);
   e->opsI_same_all = true;
   for (int i = 0; i < n; ++i) e->opsI_same_all = e->opsI_same_all && !lb_outfyb(p[i]);
+  for (int i = 0; i < n; ++i) e->general = e->general || !short_forms(p[i]);
   for (int i = 0; i < n; ++i) {
     e->m[i].init(p[i]);
     e->slotbase[i] = (int32_t)e->nslots;

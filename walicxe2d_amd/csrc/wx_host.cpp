@@ -74,7 +74,7 @@ struct wx_ctx : Mesh, Runtime {
   double *cur_u() { return U[cur].ptr; }
   double *other_u() { return U[cur ^ 1].ptr; }
   int nleaf() const { return (int)leaves.size(); }
-  QueueRef queue() const { return QueueRef{tQ, tLeaves, tLeafCap}; }
+  QueueRef queue() const { return QueueRef{tQ, tLeaves, tLeafCap, !short_forms(p), nullptr}; }
 };
 
 namespace {

@@ -295,6 +295,8 @@ __device__ __forceinline__ int flux_sweep_mild(const wx_params *__restrict__ p, 
     else ok = flux_sweep_short<NEQ, CHOICE, BS, 2, 2>(p, wave, prim, cs, F, G, fx);
   }
   if (!WX_RARE(!__all(ok))) return 0;
+  // (with the solver and limiter compiled in here as well, stage B spills: 81
+  // registers with five variables, a wave per SIMD less with six)
   return flux_sweep_t<NEQ, CHOICE, BS>(p, wave, prim, F, G, fx);
 }
 
@@ -1444,6 +1446,9 @@ int launch_slot_scatter(const SlotOps *src, int n, int2 *ops, int32_t *flag, hip
 // short: stage A at 1 174 blocks 13.9 / 13.0, at 532 7.8 / 8.2, on 19 250
 // 138 / 122; stage B at 520 11.9 / 13.1, at 1 177 19.6 / 20.2, at 5 319
 // 58.4 / 54.2, at 19 250 206 / 191.
+// Where the run's constants lie outside the short forms' range no block is
+// served by them (QueueRef::general): stages A and B of 6 144 blocks took 58 and
+// 81 us so, 46 and 65 in the general form.
 constexpr int kMildA = 1024, kMildB = 3000;
 
 int launch_stageA(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const double *U,
@@ -1454,7 +1459,7 @@ int launch_stageA(const wx_params *P, int neq, QueueRef q, int grid, int bs, int
     WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageA_dt<N>), dim3(grid), dim3(512), 0, stream, P, q, U, Q, Pc, S));
     return hip_status();
   }
-  if (!persist && grid >= kMildA) {
+  if (!persist && !q.general && grid >= kMildA) {
     WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageA_mild<N, B>), dim3(grid), dim3(B), 0, stream, P, q, U, Q, Pc, S)));
     return hip_status();
   }
@@ -1465,7 +1470,7 @@ int launch_stageA(const wx_params *P, int neq, QueueRef q, int grid, int bs, int
 int launch_stageB(const wx_params *P, int neq, QueueRef q, int grid, int bs, int persist, const int2 *ops,
                   const BlockRec *binfo, double *U, double *Q, DevScalars *S, hipStream_t stream) {
   if (grid <= 0) return WX_OK;
-  if (!persist && grid >= kMildB) {
+  if (!persist && !q.general && grid >= kMildB) {
     WX_BS_DISPATCH(bs, WX_DISPATCH(neq, hipLaunchKernelGGL((k_stageB_mild<N, B>), dim3(grid), dim3(B), 0, stream, P, q, ops, binfo, U, Q, Q, S)));
     return hip_status();
   }
