@@ -173,7 +173,7 @@ static void info_of_an_unchecked_tree() {
 // A download, of any size, reads the state and nothing else of it: no launch
 // writes the tiles, and two threads may download one context at once.
 static void downloads() {
-  for (int n : {1, 4, 80, 81, 82, 2700}) {   // states below and above 1 MiB (12.8 KB a block), and above 32 MiB
+  for (int n : {1, 4, 80, 2700}) {   // one piece, and two (12.8 KB a block, 32 MiB)
     wx_params p = params(n, 1, 1, n, 0);
     wx_ctx *c = context(p);
     Tree t = tree(c);

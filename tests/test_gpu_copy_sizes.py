@@ -1,6 +1,6 @@
-"""States at the edges of the copy paths (through pinned memory up to 1 MiB,
-downloads in pieces of 32 MiB above): up and down unchanged, every cell of the
-padded tiles, and the primitives of a state at rest."""
+"""States up and down unchanged, every cell of the padded tiles, at the edges of
+the pieces of 32 MiB that a download goes by, and the primitives of a state at
+rest."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 # 12 800 bytes a block of four variables, 16 000 of five; block 0 is copied too
-@pytest.mark.parametrize("neq,n", [(4, 1), (4, 80), (4, 81), (5, 64), (5, 65), (4, 2620), (4, 2621), (5, 4500)])
+@pytest.mark.parametrize("neq,n", [(4, 1), (5, 64), (4, 2620), (4, 2621), (5, 4500)])
 def test_round_trip(neq, n):
     cfg = P.config_c1(neq=neq, nbrootx=n, nbrooty=1, cooling="H" if neq >= 5 else "ADIABATIC", nblocks=n + 1)
     sim = Simulation(cfg)

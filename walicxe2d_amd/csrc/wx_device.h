@@ -219,9 +219,8 @@ int launch_meshops(const wx_params *P, int neq, const MeshOp *ops, int nops, dou
 // launch for all: a kernel reads the pinned staging directly.
 int launch_h2d(const CopyDesc *d, int n, hipStream_t stream);
 // mode 0: Fortran layout (src) to cap device tiles (dst, from block 1 on); 1:
-// back; cap tiles from the given ones on, tile by tile (src may be dst, either
-// may be mapped host memory): 2: padded host rows to the device's cell order,
-// 3: back.
+// back; cap tiles from the given ones on, tile by tile (src may be dst): 2:
+// padded host rows to the device's cell order, 3: back.
 int launch_transpose(int neq, int cap, const double *src, double *dst, int mode, int ld,
                      hipStream_t stream);
 

@@ -1357,9 +1357,8 @@ __global__ void k_transpose(int cap, const double *__restrict__ src, double *__r
 }
 
 // The cells of one tile variable per 128 threads reordered, between padded
-// host rows and the device's order; src may be dst.  Either side can be mapped
-// host memory: both are read and written in the order of memory, the tile
-// turned over in LDS.
+// host rows and the device's order; src may be dst.  Both are read and written
+// in the order of memory, the tile turned over in LDS.
 __global__ __launch_bounds__(256) void k_reorder(size_t ntile, const double *src, double *dst, int to_rows) {
   __shared__ double t[2][NC];
   const int h = threadIdx.x >> 7, l = threadIdx.x & 127;

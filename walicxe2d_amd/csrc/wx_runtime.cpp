@@ -7,6 +7,30 @@
 
 namespace wx {
 
+int Runtime::create_stream() {
+  if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) {
+    stream = nullptr;
+    return fail(WX_EHIP, "hipStreamCreate failed");
+  }
+  return WX_OK;
+}
+
+void Runtime::destroy() {
+  if (stream) (void)hipStreamSynchronize(stream);
+  for (auto &st : stage) {
+    if (st.ev) (void)hipEventDestroy(st.ev);
+    if (st.buf) (void)hipHostFree(st.buf);
+    if (st.hdesc) (void)hipHostFree(st.hdesc);
+    st = Stage{};
+  }
+  xtiles.release();
+  prof_collect(this);
+  for (auto e : evpool) (void)hipEventDestroy(e);
+  evpool.clear();
+  if (stream) (void)hipStreamDestroy(stream);
+  stream = nullptr;
+}
+
 // Mapped, coherent pinned memory and its device alias.
 static int pinned_alloc(size_t bytes, char **host, char **dev) {
   *host = *dev = nullptr;
@@ -20,48 +44,6 @@ static int pinned_alloc(size_t bytes, char **host, char **dev) {
     return fail(WX_EHIP, "device alias of the pinned staging");
   }
   return WX_OK;
-}
-
-// States up to this size cross the link in the reorder kernel itself, through
-// pinned memory that the calling thread fills or empties; above, the runtime's
-// copy of pageable memory is as fast (us per download / upload, so and with a
-// copy beside the kernel: 140 KB 20 / 25 and 31 / 32, 1 MB 59 / 56 and 69 / 64,
-// 2 MB 118 / 91 and 126 / 93; a copy alone of rows that need no reordering: 16 /
-// 20, 53 / 50, 110 / 79).
-constexpr size_t kXferDirect = 1 << 20;
-// Larger downloads go by pieces of this size, so that the device memory they
-// need besides the state is bounded (128 MB in ms by pieces of 4 / 8 / 32 / 64
-// MiB: 8.2 / 7.8 / 7.5 / 7.4).
-constexpr size_t kXferPiece = (size_t)32 << 20;
-
-int Runtime::create_stream() {
-  if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) {
-    stream = nullptr;
-    return fail(WX_EHIP, "hipStreamCreate failed");
-  }
-  if (pinned_alloc(kXferDirect, &xhost, &xdev)) {   // small states take the other path then
-    xhost = xdev = nullptr;
-    (void)hipGetLastError();
-  }
-  return WX_OK;
-}
-
-void Runtime::destroy() {
-  if (stream) (void)hipStreamSynchronize(stream);
-  for (auto &st : stage) {
-    if (st.ev) (void)hipEventDestroy(st.ev);
-    if (st.buf) (void)hipHostFree(st.buf);
-    if (st.hdesc) (void)hipHostFree(st.hdesc);
-    st = Stage{};
-  }
-  if (xhost) (void)hipHostFree(xhost);
-  xhost = xdev = nullptr;
-  xtiles.release();
-  prof_collect(this);
-  for (auto e : evpool) (void)hipEventDestroy(e);
-  evpool.clear();
-  if (stream) (void)hipStreamDestroy(stream);
-  stream = nullptr;
 }
 
 // Opens the next staging buffer for `total` bytes (waits only if that
@@ -277,16 +259,21 @@ void WorkerPool::run(int n, const std::function<void(int)> &fn) {
   n_ = 0;
 }
 
+// A download goes by pieces of at most this size, so that the device memory it
+// needs besides the state is bounded (128 MB in ms by pieces of 4 / 8 / 32 / 64
+// MiB: 8.2 / 7.8 / 7.5 / 7.4).
+//
+// Small states through mapped pinned memory, with the reorder kernel on one side
+// of the link and the calling thread on the other, were faster by themselves (16
+// blocks of five variables 25 us down and 28 up, against 38 and 37 with a copy
+// beside the kernel) but not in a run: a pass of 16 blocks, upload, 200 steps
+// and download, took 3.83 ms against 3.77, because the first fifty steps after
+// such a copy take up to twice as long to launch.
+constexpr size_t kXferPiece = (size_t)32 << 20;
+
 int tiles_to_host(Runtime *r, const double *tiles, size_t ntile, int neq, double *host) {
   std::lock_guard<std::mutex> lk(r->xmu);
-  const size_t tile = (size_t)neq * NC, bytes = ntile * tile * sizeof(double);
-  if (bytes <= kXferDirect && r->xhost) {
-    const int rc = launch_transpose(neq, (int)ntile, tiles, (double *)r->xdev, 3, 0, r->stream);
-    if (rc) return fail(rc, "reorder launch failed");
-    HIPCHK(hipStreamSynchronize(r->stream));
-    memcpy(host, r->xhost, bytes);
-    return WX_OK;
-  }
+  const size_t tile = (size_t)neq * NC;
   size_t per = std::min(ntile, std::max<size_t>(1, kXferPiece / (tile * sizeof(double))));
   int rc;
   while ((rc = r->xtiles.ensure(per * tile)) && per > 1) {   // little memory left: smaller pieces
@@ -307,16 +294,8 @@ int tiles_to_host(Runtime *r, const double *tiles, size_t ntile, int neq, double
 }
 
 int tiles_to_device(Runtime *r, const double *host, size_t ntile, int neq, double *tiles) {
-  const size_t bytes = ntile * neq * NC * sizeof(double);
-  const bool direct = bytes <= kXferDirect && r->xhost;
-  std::unique_lock<std::mutex> lk(r->xmu, std::defer_lock);
-  if (direct) {
-    lk.lock();
-    memcpy(r->xhost, host, bytes);
-  } else {
-    HIPCHK(hipMemcpyAsync(tiles, host, bytes, hipMemcpyHostToDevice, r->stream));
-  }
-  const int rc = launch_transpose(neq, (int)ntile, direct ? (const double *)r->xdev : tiles, tiles, 2, 0, r->stream);
+  HIPCHK(hipMemcpyAsync(tiles, host, ntile * neq * NC * sizeof(double), hipMemcpyHostToDevice, r->stream));
+  const int rc = launch_transpose(neq, (int)ntile, tiles, tiles, 2, 0, r->stream);
   if (rc) return fail(rc, "reorder launch failed");
   HIPCHK(hipStreamSynchronize(r->stream));
   return WX_OK;

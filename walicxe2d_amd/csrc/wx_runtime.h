@@ -199,10 +199,8 @@ struct Runtime {
   double prof_ms[NPROF] = {0};
   int64_t prof_n[NPROF] = {0};
 
-  // What state copies pass through (tiles_to_host, tiles_to_device): mapped
-  // pinned memory for small ones, device memory for a piece of a large
-  // download.  A download changes nothing but these, so it takes the lock.
-  char *xhost = nullptr, *xdev = nullptr;
+  // A piece of a download (tiles_to_host), as padded rows.  A download changes
+  // nothing but this, so it takes the lock.
   DevBuf<double> xtiles;
   std::mutex xmu;
 
