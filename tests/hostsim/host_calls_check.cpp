@@ -231,6 +231,22 @@ static void general_form() {
   }
 }
 
+// wx_profile counts the dt reduction where it is a launch (above 512 leaves),
+// not where stage A takes it.
+static void profile_counts() {
+  for (int rx : {32, 33}) {   // 512 and 528 roots
+    wx_ctx *c = context(params(rx, 16, 1, rx * 16, 0));
+    double ms[wx::NPROF], t, dt, z;
+    int64_t n[wx::NPROF];
+    REQUIRE(wx_profile(c, 1, ms, n, wx::NPROF) == WX_OK);
+    REQUIRE(wx_step(c, 3, 0, &t, &dt, &z) == WX_OK);
+    REQUIRE(wx_profile(c, -1, ms, n, wx::NPROF) == WX_OK);
+    REQUIRE(n[wx::KID_STAGEA] == 3 && n[wx::KID_STAGEB] == 3 && n[wx::KID_FILLI] == 3);
+    REQUIRE(n[wx::KID_DTRED] == (rx == 32 ? 0 : 3));
+    wx_destroy(c);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "rejected_list") rejected_list();
@@ -238,6 +254,7 @@ int main(int argc, char **argv) {
   else if (what == "info_of_an_unchecked_tree") info_of_an_unchecked_tree();
   else if (what == "downloads") downloads();
   else if (what == "general_form") general_form();
+  else if (what == "profile_counts") profile_counts();
   else return 2;
   return 0;
 }

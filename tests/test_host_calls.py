@@ -60,3 +60,7 @@ def test_downloads_only_read(program, program_tsan):
 
 def test_general_form_of_the_stages(program):
     _run(program, "general_form")
+
+
+def test_profile_counts_launches(program):
+    _run(program, "profile_counts")

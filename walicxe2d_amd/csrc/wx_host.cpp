@@ -824,7 +824,7 @@ int wx_step(wx_ctx *c, int32_t nsteps, int32_t do_admesh_flag, double *time, dou
     if (rc) return rc;
     const bool few = c->nleaf() >= 1 && c->nleaf() <= kFewLeaves;
     {
-      ProfScope ps(c, KID_DTRED);      // timestep; time += dt
+      ProfScope ps(c, few ? -1 : KID_DTRED);   // timestep; time += dt (no launch where stage A takes it)
       rc = launch_dtreduce(c->dP.ptr, c->tLeaves, c->dStat.ptr, c->tOff, 1, c->dS.ptr, few ? kDtInStageA : 1,
                            c->stream);
     }
