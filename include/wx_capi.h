@@ -96,7 +96,9 @@ int wx_upload(wx_ctx *ctx, const double *u, int32_t layout, const int32_t *lp,
  * writes tiles 0..nbmax; WX_LAYOUT_FORTRAN writes ld block rows (ld >= nbmax,
  * the host array's leading dimension; ld <= 0 means nbmax).  The reference
  * reads its arrays in place, so this is the transpose out of the device tiles
- * that output.f90 (src/output.f90:39-67) needs before it writes. */
+ * that output.f90 (src/output.f90:39-67) needs before it writes.  In
+ * WX_LAYOUT_BLOCK without prim two host threads may download one context at
+ * once: the state is only read. */
 int wx_download(wx_ctx *ctx, double *u, double *prim, int32_t layout, int32_t ld);
 /* Device -> host copy of the mesh tree kept by the context's own admesh. */
 int wx_get_tree(wx_ctx *ctx, int32_t *lp, int32_t *leaf, int32_t *icoord, int32_t ld,
